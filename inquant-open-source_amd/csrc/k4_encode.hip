@@ -8,6 +8,7 @@
 //   phase 3  scales, 4-bit slots, 8-bit salient codes split across the
 //            source and donor slots, nibble packing, padding (codec.py:218-233).
 // Results are bit-identical to the reference CPU implementation.
+#include "k4_stats_dev.h"
 #include "select_dev.h"
 #include "v_rows_dev.h"
 
@@ -49,9 +50,6 @@ struct K4Args {
     // of v are encoded group-wise into the outputs of iq_v_quantize
     uint8_t *vpayload;
     uint16_t *vscales, *voffsets;
-    // k4_encode_kernel with long rows: statistics, selection, scales and
-    // descriptors only; k4_quantize_generic then writes the payload
-    int split;
 };
 
 __device__ __forceinline__ void store_desc(void *p, int64_t i, int v, int bytes)
@@ -61,7 +59,6 @@ __device__ __forceinline__ void store_desc(void *p, int64_t i, int v, int bytes)
     else ((int64_t *)p)[i] = v;
 }
 
-// Sampled sums of one channel in torch's order (cascade, or interleaved row_sum).
 // Calls f(v, i) for i = 0 .. n - 1 in order with v the element at
 // base + (i * mul + add) * step, loading SEQ_PF elements ahead of their use
 // (one memory round trip per SEQ_PF elements of a sequential reduction).
@@ -129,29 +126,20 @@ __device__ __forceinline__ double iq_read_lane_f64(double v, int l)
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
-template <typename F>
-__device__ __forceinline__ void for_each_seq(const void *x, int dt, int64_t base, int64_t step, int64_t n, int64_t mul,
-                                             int64_t add, F &&f)
-{
-    switch (dt) {
-    case IQ_BF16: for_each_seq_t<IQ_BF16>(x, base, step, n, mul, add, f); break;
-    case IQ_F16: for_each_seq_t<IQ_F16>(x, base, step, n, mul, add, f); break;
-    case IQ_F64: for_each_seq_t<IQ_F64>(x, base, step, n, mul, add, f); break;
-    default: for_each_seq_t<IQ_F32>(x, base, step, n, mul, add, f); break;
-    }
-}
-
-__device__ __forceinline__ void sampled_sums(const void *x, int dt, int64_t base, int64_t step, int64_t ns, bool cascade_col,
-                             float &sum_abs, float &sum)
+// Sampled sums of one channel in torch's order (cascade, or interleaved row_sum).
+template <int DT>
+__device__ __forceinline__ void sampled_sums(const void *x, int64_t base, int64_t step, int64_t ns, bool cascade_col,
+                                             float &sum_abs, float &sum)
 {
     if (cascade_col) {
         IqCascade a, s;
         a.init(ns);
         s.init(ns);
-        for_each_seq(x, dt, base, step, ns, 1, 0, [&](float v, int64_t) {
+        auto f = [&](float v, int64_t) {
             a.add(fabsf(v));
             s.add(v);
-        });
+        };
+        for_each_seq_t<DT>(x, base, step, ns, 1, 0, f);
         sum_abs = a.finish();
         sum = s.finish();
     } else {
@@ -161,15 +149,16 @@ __device__ __forceinline__ void sampled_sums(const void *x, int dt, int64_t base
             IqCascade a, s;
             a.init(g);
             s.init(g);
-            for_each_seq(x, dt, base, step, g, 4, k, [&](float v, int64_t) {
+            auto f = [&](float v, int64_t) {
                 a.add(fabsf(v));
                 s.add(v);
-            });
+            };
+            for_each_seq_t<DT>(x, base, step, g, 4, k, f);
             pa[k] = a.finish();
             ps[k] = s.finish();
         }
         for (int64_t r = 4 * g; r < ns; ++r) {
-            const float v = iq_load_f32(x, base + r * step, dt);
+            const float v = iq_load_f32(x, base + r * step, DT);
             pa[0] = __fadd_rn(pa[0], fabsf(v));
             ps[0] = __fadd_rn(ps[0], v);
         }
@@ -178,158 +167,218 @@ __device__ __forceinline__ void sampled_sums(const void *x, int dt, int64_t base
     }
 }
 
-__global__ __launch_bounds__(K4_THREADS) void k4_encode_kernel(K4Args a)
+template <bool F16IN>
+__device__ __forceinline__ float tile_f32(uint32_t bits16)
 {
-    __shared__ float s_sal[IQ_MAXD];
-    __shared__ float s_smean[IQ_MAXD];
-    __shared__ float s_err[IQ_MAXD];
-    __shared__ float s_scale[IQ_MAXD];
-    __shared__ int16_t s_src_of[IQ_MAXD];
-    __shared__ uint8_t s_is_src[IQ_MAXD];
-    __shared__ int16_t s_src[IQ_MAXD / 2];
-    __shared__ int16_t s_don[IQ_MAXD / 2];
-    __shared__ int s_bad;
+    if constexpr (F16IN) return iq_f16_to_f32((uint16_t)bits16);
+    else return __uint_as_float(bits16 << 16);
+}
 
-    const int tid = threadIdx.x;
-    const int64_t row = blockIdx.x;
-    const int64_t b = row / a.H, h = row % a.H;
-    const int64_t base = b * a.sb + h * a.sh;
-    const int64_t T = a.T, D = a.D;
-    const int64_t ns = (T + a.stride - 1) / a.stride;
-    const int64_t ncasc = iq_cascade_columns(D);
+// ---------------------------------------------------------------------------
+// General rows: any dtype, stride, length and (even) head size.  A row of up
+// to LONG_ROW tokens is one workgroup's (k4_encode_kernel); a longer one is
+// spread over the chip in three launches (k4_row_stats, k4_row_select,
+// k4_quantize_rows).  Both take the donor errors from order-free sums with a
+// certificate (k4_stats_dev.h), so nothing but the saliency sums has an order
+// to keep, and torch's cascade leaves those in independent pieces.  Eight rows
+// of 32768 bf16 tokens x 128 channels: 22.7 + 16.4 + 21.8 us (3.0, then 3.8
+// TB/s of rows read and words written; 3390 + 89 us with a sequential fp64
+// chain per channel); four of 4096: 6.3 + 12.3 + 6.4 us (342 + 23).  The
+// second launch is latency: a few workgroups, one after the other the partial
+// results' round trips, the radix selections and the picks.
+constexpr int ROW_THREADS = 512;
+constexpr int ROW_WAVES = ROW_THREADS / 64;
+constexpr int ROW_GROUPS = ROW_WAVES / 2;
+// Two rows of 64 fp16 channels take 17.4 us in one workgroup each and 18.3
+// spread at 256 tokens, 19.9 and 18.5 at 384, 51 and 19 at 2048; 512 rows 35
+// and 37 at 256 tokens, 46 and 44 at 512.
+constexpr int64_t LONG_ROW = 256;
 
-    if (tid == 0) s_bad = 0;
-    __syncthreads();
+struct RowLds {
+    float sal[IQ_MAXD], smean[IQ_MAXD], err[IQ_MAXD], ehi[IQ_MAXD], scale[IQ_MAXD];
+    int16_t src_of[IQ_MAXD], src[IQ_MAXD / 2], don[IQ_MAXD / 2], list[64];
+    uint8_t is_src[IQ_MAXD];
+    int bad, again;
+};
 
-    // ---- phase 1: per-channel statistics (one thread per channel).  Every
-    // lane of a wave that has channels left runs the loop (lanes past D repeat
-    // channel D - 1 and write nothing), so the reciprocals that lanes compute
-    // for each other below are always there to read.
-    const int lane = tid & 63;
-    for (int64_t c0 = tid - lane; c0 < D; c0 += K4_THREADS) {
-        const bool own = c0 + lane < D;
-        const int64_t c = own ? c0 + lane : D - 1;
-        const int64_t cb = base + c * a.sc;
-        float sum_abs, sum;
-        sampled_sums(a.x, a.dt, cb, a.st * a.stride, ns, c < ncasc, sum_abs, sum);
-        const float smean = sum / (float)ns;
-        if (own) {
-            s_sal[c] = sum_abs / (float)ns;
-            s_smean[c] = smean;
+// Partial sums of 64 channels by one wavefront.
+struct RowPart {
+    double s1[64], s2[64];
+    float amax[64];
+};
+
+// Sums, largest magnitude and finiteness of one channel's tokens t0, t0 +
+// step, ... < t1, sixteen loads in flight.
+template <int DT>
+__device__ __forceinline__ void stats_slice(const void *x, int64_t cb, int64_t st, int64_t t0, int64_t t1, int64_t step,
+                                            double &s1, double &s2, float &amax, bool &bad)
+{
+    s1 = s2 = 0.0;
+    amax = 0.0f;
+    bad = false;
+    constexpr int U = 16;
+    for (int64_t t = t0; t < t1; t += U * step) {
+        float v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t tt = t + u * step;
+            v[u] = iq_load_f32(x, cb + (tt < t1 ? tt : t0) * st, DT);
         }
-        float amax = 0.0f;
-        bool bad = false;
-        double mean = 0.0, m2 = 0.0, ygrp = 0.0;
-        const bool me = a.min_error;
-        // rows of up to 2^24 tokens take the reciprocal from iq_rcp_small_int
-        auto stats = [&](auto small) {
-            for_each_seq(a.x, a.dt, cb, a.st, T, 1, 0, [&](float v, int64_t t) {
-            bad |= !iq_isfinite(v);
-            amax = fmaxf(amax, fabsf(v));
-            if (me) {
-                // delta / n as RN(1 / n) (off the dependent chain) and one
-                // remainder correction: the correctly rounded quotient
-                // (tests/test_welford_division.py, n up to 2^24)
-                const double n = decltype(small)::value ? (double)(uint32_t)(t + 1) : (double)(t + 1);
-                // rows of up to 2^24 tokens: at the start of each group of
-                // SEQ_PF steps (t a multiple of SEQ_PF there, for_each_seq_t's
-                // groups) lane l computes RN(1 / (t + 1 + l % SEQ_PF)), and
-                // step t reads it from lane t % SEQ_PF: one reciprocal per
-                // group instead of one per step
-                double y;
-                if constexpr (decltype(small)::value) {
-                    if ((t & (SEQ_PF - 1)) == 0) ygrp = iq_rcp_small_int((uint32_t)(t + 1 + (lane & (SEQ_PF - 1))));
-                    y = iq_read_lane_f64(ygrp, (int)(t & (SEQ_PF - 1)));
-                } else {
-                    y = 1.0 / n;
-                }
-                const double dv = (double)v;
-                const double delta = __dsub_rn(dv, mean);
-                const double q0 = __dmul_rn(delta, y);
-                const double r = __builtin_fma(-q0, n, delta);
-                mean = __dadd_rn(mean, __builtin_fma(r, y, q0));
-                const double nd = __dsub_rn(dv, mean);
-                m2 = __dadd_rn(m2, __dmul_rn(delta, nd));
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (t + u * step >= t1) v[u] = 0.0f;
+            bad |= !iq_isfinite(v[u]);
+            amax = fmaxf(amax, fabsf(v[u]));
+            const double d = (double)v[u];
+            s1 = __dadd_rn(s1, d);
+            s2 = __builtin_fma(d, d, s2);
+        }
+    }
+}
+
+// The reference's donor error of one channel by its sequential fp64 Welford
+// chain (rows whose pool the order-free sums leave uncertain).  Every lane of
+// the wavefront runs it (lanes past D repeat the last channel).
+template <int DT>
+__device__ __forceinline__ float welford_error(const void *x, int64_t cb, int64_t st, int64_t T, float smean)
+{
+    const int lane = threadIdx.x & 63;
+    double mean = 0.0, m2 = 0.0, ygrp = 0.0;
+    auto chain = [&](auto small) {
+        auto f = [&](float v, int64_t t) {
+            // delta / n as RN(1 / n) (off the dependent chain) and one
+            // remainder correction: the correctly rounded quotient
+            // (tests/test_welford_division.py, n up to 2^24)
+            const double n = decltype(small)::value ? (double)(uint32_t)(t + 1) : (double)(t + 1);
+            // rows of up to 2^24 tokens: at the start of each group of
+            // SEQ_PF steps (t a multiple of SEQ_PF there, for_each_seq_t's
+            // groups) lane l computes RN(1 / (t + 1 + l % SEQ_PF)), and
+            // step t reads it from lane t % SEQ_PF: one reciprocal per
+            // group instead of one per step
+            double y;
+            if constexpr (decltype(small)::value) {
+                if ((t & (SEQ_PF - 1)) == 0) ygrp = iq_rcp_small_int((uint32_t)(t + 1 + (lane & (SEQ_PF - 1))));
+                y = iq_read_lane_f64(ygrp, (int)(t & (SEQ_PF - 1)));
+            } else {
+                y = 1.0 / n;
             }
-            });
+            const double dv = (double)v;
+            const double delta = __dsub_rn(dv, mean);
+            const double q0 = __dmul_rn(delta, y);
+            const double r = __builtin_fma(-q0, n, delta);
+            mean = __dadd_rn(mean, __builtin_fma(r, y, q0));
+            const double nd = __dsub_rn(dv, mean);
+            m2 = __dadd_rn(m2, __dmul_rn(delta, nd));
         };
-        if (T <= (int64_t(1) << 24)) stats(std::true_type{});
-        else stats(std::false_type{});
-        if (a.min_error) {
-            const float var = (float)(m2 / (double)T);
-            const float diff = __fsub_rn((float)mean, smean);
-            if (own) s_err[c] = __fadd_rn(var, __fmul_rn(diff, diff));
-        }
-        if (own) s_scale[c] = amax;
-        if (bad) s_bad = 1;
+        for_each_seq_t<DT>(x, cb, st, T, 1, 0, f);
+    };
+    if (T <= (int64_t(1) << 24)) chain(std::true_type{});
+    else chain(std::false_type{});
+    const float var = (float)(m2 / (double)T);
+    const float diff = __fsub_rn((float)mean, smean);
+    return __fadd_rn(var, __fmul_rn(diff, diff));
+}
+
+// The selection on the sequential errors, for rows whose pool is uncertain.
+// A call of its own: inlined, its registers and hoisted address arithmetic cost
+// the rows that never need it 6 us of 18 (one 256-token row a workgroup).
+template <int DT, bool WIDE>
+__device__ __attribute__((noinline)) void select_sequential(const void *x, int64_t base, int64_t sc, int64_t st, int64_t T,
+                                                            int D, int count, RowLds *s)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    for (int c0 = tid - lane; c0 < D; c0 += ROW_THREADS) {
+        const int c = min(c0 + lane, D - 1);
+        const float e = welford_error<DT>(x, base + c * sc, st, T, s->smean[c]);
+        if (c0 + lane < D) s->err[c] = e;
     }
     __syncthreads();
+    if (tid < 64) iq_select_wave<WIDE>(s->sal, s->err, D, count, s->src, s->don, s->is_src, s->src_of);
+}
 
-    // ---- phase 2: selection by wavefront 0
+// Selection, scales, descriptors and padding of a row whose statistics are in
+// LDS (s.scale holds the largest magnitudes; a barrier behind them).  Every
+// thread of the workgroup calls it; it ends with a barrier.  WIDE: D > 256
+// (the selection's lane masks of 512 and 1024 channels spill registers, which
+// the narrower rows' kernels should not carry).
+template <int DT, bool WIDE>
+__device__ __forceinline__ void row_select(const K4Args &a, RowLds &s, int64_t row, int64_t base)
+{
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int64_t D = a.D;
     if (tid < 64) {
-        iq_select_wave(s_sal, a.min_error ? s_err : nullptr, (int)D, (int)a.count, s_src, s_don, s_is_src,
-                       s_src_of);
+        const float *err = a.min_error ? s.err : nullptr;
+        if (!WIDE && D == 128) iq_select_wave128(s.sal, err, (int)a.count, s.src, s.don, s.is_src, s.src_of, s.list);
+        else iq_select_wave<WIDE>(s.sal, err, (int)D, (int)a.count, s.src, s.don, s.is_src, s.src_of);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const bool again = a.min_error && !s.bad && !iq_pool_certain(s.err, s.ehi, (int)D, s.is_src, s.src_of);
+        if (lane == 0) s.again = again;
     }
     __syncthreads();
-
-    // ---- scales and descriptors
+    if (s.again) {
+        select_sequential<DT, WIDE>(a.x, base, a.sc, a.st, a.T, (int)D, (int)a.count, &s);
+        __syncthreads();
+    }
     const float flt_min = 1.17549435e-38f;
-    for (int64_t c = tid; c < D; c += K4_THREADS) {
-        const float s = s_scale[c] / (s_is_src[c] ? 127.0f : 7.0f);
-        const float sc = s < flt_min ? flt_min : s;
-        s_scale[c] = sc;
+    for (int64_t c = tid; c < D; c += ROW_THREADS) {
+        const float q = s.scale[c] / (s.is_src[c] ? 127.0f : 7.0f);
+        const float sc = q < flt_min ? flt_min : q;
+        s.scale[c] = sc;
         a.scales[row * D + c] = sc;
     }
-    for (int64_t i = tid; i < a.count; i += K4_THREADS) {
-        store_desc(a.src, row * a.count + i, s_src[i], a.desc_bytes);
-        store_desc(a.don, row * a.count + i, s_don[i], a.desc_bytes);
-        a.padding[row * a.count + i] = s_smean[s_don[i]];
+    for (int64_t i = tid; i < a.count; i += ROW_THREADS) {
+        store_desc(a.src, row * a.count + i, s.src[i], a.desc_bytes);
+        store_desc(a.don, row * a.count + i, s.don[i], a.desc_bytes);
+        a.padding[row * a.count + i] = s.smean[s.don[i]];
     }
-    if (tid == 0 && s_bad) atomicOr(a.bad, 1);
+    if (tid == 0 && s.bad) atomicOr(a.bad, 1);
     __syncthreads();
+}
 
-    if (a.split) return;
-
-    // ---- phase 3: slots and nibble packing, one payload byte per step, the
-    // inputs of P3_UNROLL steps loaded before any is used
-    const int64_t half = D / 2;
-    uint8_t *out = a.payload + row * T * half;
+// The 4-bit slots of a row's tokens [t0, t1), one payload byte per step, the
+// inputs of P3_UNROLL steps loaded before any is used: any layout.
+template <int DT, int NT>
+__device__ __forceinline__ void quantize_bytes(const K4Args &a, const float *scale, const uint8_t *is_src,
+                                               const int16_t *src_of, int64_t row, int64_t base, int64_t t0, int64_t t1)
+{
+    const int64_t half = a.D / 2;
+    uint8_t *out = a.payload + row * a.T * half;
     constexpr int P3_UNROLL = 8;
-    for (int64_t idx0 = tid; idx0 < T * half; idx0 += (int64_t)K4_THREADS * P3_UNROLL) {
+    for (int64_t idx0 = t0 * half + threadIdx.x; idx0 < t1 * half; idx0 += (int64_t)NT * P3_UNROLL) {
         float xv[P3_UNROLL][2];
 #pragma unroll
         for (int u = 0; u < P3_UNROLL; ++u) {
-            const int64_t idx = idx0 + (int64_t)u * K4_THREADS;
-            const int64_t ic = idx < T * half ? idx : T * half - 1;
+            const int64_t idx = idx0 + (int64_t)u * NT;
+            const int64_t ic = idx < t1 * half ? idx : t1 * half - 1;
             const int64_t t = ic / half, j = ic - t * half;
             const int64_t tb = base + t * a.st;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const int64_t c = 2 * j + e;
-                const int16_t owner = s_src_of[c];
-                const int64_t sc = (s_is_src[c] || owner < 0) ? c : owner;    // the channel slot c encodes
-                xv[u][e] = iq_load_f32(a.x, tb + sc * a.sc, a.dt);
+                const int16_t owner = src_of[c];
+                const int64_t sc = (is_src[c] || owner < 0) ? c : owner;    // the channel slot c encodes
+                xv[u][e] = iq_load_f32(a.x, tb + sc * a.sc, DT);
             }
         }
 #pragma unroll
         for (int u = 0; u < P3_UNROLL; ++u) {
-            const int64_t idx = idx0 + (int64_t)u * K4_THREADS;
-            if (idx >= T * half) break;
+            const int64_t idx = idx0 + (int64_t)u * NT;
+            if (idx >= t1 * half) break;
             const int64_t j = idx % half;
             uint32_t slots[2];
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const int64_t c = 2 * j + e;
-                const int16_t owner = s_src_of[c];
+                const int16_t owner = src_of[c];
                 float q;
-                if (s_is_src[c] || owner >= 0) {
-                    const int64_t sc = s_is_src[c] ? c : owner;
-                    q = rintf(xv[u][e] / s_scale[sc]);
+                if (is_src[c] || owner >= 0) {
+                    const int64_t sc = is_src[c] ? c : owner;
+                    q = rintf(xv[u][e] / scale[sc]);
                     q = fminf(fmaxf(q, -127.0f), 127.0f);
                     const uint32_t code = (uint32_t)(q + 128.0f);
-                    slots[e] = s_is_src[c] ? (code >> 4) : (code & 15u);
+                    slots[e] = is_src[c] ? (code >> 4) : (code & 15u);
                 } else {
-                    q = rintf(xv[u][e] / s_scale[c]);
+                    q = rintf(xv[u][e] / scale[c]);
                     q = fminf(fmaxf(q, -7.0f), 7.0f);
                     slots[e] = (uint32_t)(q + 8.0f);
                 }
@@ -337,117 +386,6 @@ __global__ __launch_bounds__(K4_THREADS) void k4_encode_kernel(K4Args a)
             out[idx] = (uint8_t)(slots[0] | (slots[1] << 4));
         }
     }
-}
-
-// Phase 3 of k4_encode_kernel for long rows, spread over the tokens: grid
-// (token tiles of Q_TOKENS, rows); each workgroup takes the row's scales and
-// descriptors from global memory (written by the statistics launch) and
-// quantizes its tokens exactly as phase 3 does.
-constexpr int64_t Q_TOKENS = 64;
-
-__global__ __launch_bounds__(K4_THREADS) void k4_quantize_generic(K4Args a)
-{
-    __shared__ float s_scale[IQ_MAXD];
-    __shared__ int16_t s_src_of[IQ_MAXD];
-    __shared__ uint8_t s_is_src[IQ_MAXD];
-    const int tid = threadIdx.x;
-    const int64_t row = blockIdx.y, b = row / a.H, h = row % a.H;
-    const int64_t base = b * a.sb + h * a.sh, D = a.D, half = D / 2;
-    auto desc = [&](const void *p, int64_t i) -> int {
-        return a.desc_bytes == 1 ? ((const uint8_t *)p)[i]
-               : a.desc_bytes == 4 ? ((const int32_t *)p)[i] : (int)((const int64_t *)p)[i];
-    };
-    for (int64_t c = tid; c < D; c += K4_THREADS) {
-        s_scale[c] = a.scales[row * D + c];
-        s_is_src[c] = 0;
-        s_src_of[c] = -1;
-    }
-    __syncthreads();
-    for (int64_t i = tid; i < a.count; i += K4_THREADS) {
-        const int sc = desc(a.src, row * a.count + i), dn = desc(a.don, row * a.count + i);
-        s_is_src[sc] = 1;
-        s_src_of[dn] = (int16_t)sc;
-    }
-    __syncthreads();
-    const int64_t t0 = (int64_t)blockIdx.x * Q_TOKENS, t1 = t0 + Q_TOKENS < a.T ? t0 + Q_TOKENS : a.T;
-    uint8_t *out = a.payload + row * a.T * half;
-    for (int64_t idx = t0 * half + tid; idx < t1 * half; idx += K4_THREADS) {
-        const int64_t t = idx / half, j = idx - t * half;
-        const int64_t tb = base + t * a.st;
-        uint32_t slots[2];
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            const int64_t c = 2 * j + e;
-            const int16_t owner = s_src_of[c];
-            float q;
-            if (s_is_src[c] || owner >= 0) {
-                const int64_t sc = s_is_src[c] ? c : owner;
-                q = rintf(iq_load_f32(a.x, tb + sc * a.sc, a.dt) / s_scale[sc]);
-                q = fminf(fmaxf(q, -127.0f), 127.0f);
-                const uint32_t code = (uint32_t)(q + 128.0f);
-                slots[e] = s_is_src[c] ? (code >> 4) : (code & 15u);
-            } else {
-                q = rintf(iq_load_f32(a.x, tb + c * a.sc, a.dt) / s_scale[c]);
-                q = fminf(fmaxf(q, -7.0f), 7.0f);
-                slots[e] = (uint32_t)(q + 8.0f);
-            }
-        }
-        out[idx] = (uint8_t)(slots[0] | (slots[1] << 4));
-    }
-}
-
-// ---------------------------------------------------------------------------
-// Tile encoder for the cache shapes: D = 128, 16-bit input, T <= 256 tokens,
-// channel-contiguous rows.  The block streams through LDS in 32-token chunks
-// (double-buffered, 16-byte loads, three chunks in flight while the current
-// one is consumed), twice:
-//   pass 1  waves 0-1: the fp64 Welford var_mean of channel tid (min_error
-//           only); delta / n uses a table of RN(1/n) and one remainder fma,
-//           which is the correctly rounded quotient for n <= 256 (sealed
-//           blocks: one fma with compile-time constants, see step_c);
-//           waves 2-3: sampled sums (torch cascade order), amax and
-//           finiteness as an integer max of the 16-bit magnitudes;
-//   then    donor selection by the whole workgroup (iq_select_tile128);
-//           the sequential donor picks run on one wavefront alone, and with a
-//           value row to encode (page mode, or VB = 2 / 4) the other three
-//           group-encode the values meanwhile (v_encode16, the same bits as
-//           v_encode_rows), reading them from HBM while it is otherwise idle;
-//   pass 2  every thread quantizes 8 channels of a token per step, writing
-//           4 payload bytes.
-// LDS stays under 40 KiB, so four blocks share a compute unit and their
-// latency-bound phases (the Welford chains, the donor picks) overlap.
-// Bit-identical to k4_encode_kernel.
-constexpr int TILE_D = 128;
-constexpr int TILE_T = 256;
-constexpr int CH = 32;                   // tokens per staged chunk
-constexpr int KPF = 1;                   // chunks in flight
-constexpr int XROW = TILE_D + 8;         // u16 per staged row: 68 dwords (16-byte aligned rows, distinct banks)
-// sealed blocks stream by direct global -> LDS loads into NBUF chunk buffers
-// (unpadded rows), NBUF - 1 chunks in flight while one is processed
-constexpr int NBUF_DMA = 4;
-
-// s_waitcnt vmcnt(2 * ahead) lgkmcnt(0), then s_barrier: this wave's loads
-// of every chunk but the `ahead` newest have landed in LDS and its LDS reads
-// are done; after the barrier the same holds for every wave.  Vector memory
-// operations retire in issue order, so at most 2 * ahead outstanding means
-// every older load is done; stores issued after a chunk's loads only make
-// the wait longer.  (A plain __syncthreads would wait for all loads in
-// flight.)
-__device__ __forceinline__ void wait_chunk_barrier(int ahead)
-{
-    switch (ahead) {
-    case 0: asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
-    case 1: asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
-    case 2: asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
-    default: asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
-    }
-}
-
-template <bool F16IN>
-__device__ __forceinline__ float tile_f32(uint32_t bits16)
-{
-    if constexpr (F16IN) return iq_f16_to_f32((uint16_t)bits16);
-    else return __uint_as_float(bits16 << 16);
 }
 
 // The eight 4-bit slots of channels 8 j .. 8 j + 7 (one packed word per
@@ -520,6 +458,596 @@ struct K4Slots {
         return w;
     }
 };
+
+// quantize_bytes for channel-contiguous rows on 16-byte boundaries, D a
+// multiple of 8: a thread loads 8 channels of one token (two steps ahead of
+// their use), the step's tokens meet in LDS, where a donor slot finds its
+// source's value, and each thread packs one word.  The tile holds two steps,
+// so one barrier a step suffices.
+template <int DT, int NT>
+struct RowTile {
+    static constexpr int EB = DT == IQ_F32 ? 4 : 2;      // element bytes
+    uint8_t x[2][NT * 8 * EB];
+};
+
+template <int DT, int NT>
+__device__ __forceinline__ void quantize_words(const K4Args &a, const float *scale, const uint8_t *is_src,
+                                               const int16_t *src_of, RowTile<DT, NT> &tile, int64_t row, int64_t base,
+                                               int64_t t0, int64_t t1)
+{
+    constexpr int EB = RowTile<DT, NT>::EB, NV = EB / 2;
+    const int L = (int)a.D / 8, tps = NT / L;             // lanes per token, tokens per step
+    const int tid = threadIdx.x, tt = tid / L, j = tid - tt * L;
+    const bool live = tt < tps;
+    K4Slots slots;
+    slots.init(j, is_src, src_of, scale);
+    // 64 / L whole tokens a wavefront: it reads only what it wrote, so its
+    // own in-order LDS operations are all the synchronization
+    const bool local = 64 % L == 0;
+    const int64_t pitch = a.st * EB, step = tps * pitch;
+    const char *src = (const char *)a.x + (base + 8 * j) * EB + (t0 + tt) * pitch;
+    const char *const last = (const char *)a.x + (base + 8 * j) * EB + (t1 - 1) * pitch;
+    uint32_t *out = (uint32_t *)a.payload + (row * a.T + t0 + tt) * L + j;
+    u32x4_t cur[NV], nxt[NV], far[NV];
+    auto load = [&](const char *p, int64_t t, u32x4_t (&r)[NV]) {     // t: the token p stands on
+        const u32x4_t *q = (const u32x4_t *)(t < t1 ? p : last);
+#pragma unroll
+        for (int k = 0; k < NV; ++k) r[k] = q[k];
+    };
+    load(src, t0 + tt, cur);
+    load(src + step, t0 + tt + tps, nxt);
+    int buf = 0;
+    for (int64_t t = t0 + tt; t - tt < t1; t += tps, buf ^= 1) {
+        src += step;
+        load(src + step, t + 2 * tps, far);
+        uint8_t *xs = tile.x[buf] + tt * (int)a.D * EB;
+        if (live) {
+#pragma unroll
+            for (int k = 0; k < NV; ++k) ((u32x4_t *)(xs + 8 * j * EB))[k] = cur[k];
+        }
+        if (local) __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        else __syncthreads();
+        if (live && t < t1) {
+            float v[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = iq_load_f32(xs, slots.srcc[e], DT);
+            __builtin_nontemporal_store(slots.word(v), out);
+        }
+        out += tps * L;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+            cur[k] = nxt[k];
+            nxt[k] = far[k];
+        }
+    }
+}
+
+// WORDS: the rows take quantize_words.
+template <int DT, bool WORDS, bool WIDE>
+__global__ __launch_bounds__(ROW_THREADS) void k4_encode_kernel(K4Args a)
+{
+    __shared__ RowLds s;
+    // the statistics' partial sums, then the quantizer's tile
+    constexpr size_t PART = ROW_WAVES * sizeof(RowPart), TILE = sizeof(RowTile<DT, ROW_THREADS>);
+    __shared__ __attribute__((aligned(16))) uint8_t scratch[WORDS && TILE > PART ? TILE : PART];
+    RowPart *const part = (RowPart *)scratch;
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t row = blockIdx.x;
+    const int64_t b = row / a.H, h = row % a.H;
+    const int64_t base = b * a.sb + h * a.sh;
+    const int64_t T = a.T, D = a.D;
+    const int64_t ns = (T + a.stride - 1) / a.stride;
+    const int64_t ncasc = iq_cascade_columns(D);
+
+    if (tid == 0) s.bad = 0;
+    __syncthreads();
+
+    // ---- statistics, up to 4 groups of 64 channels at a time: a wavefront
+    // of each group takes the sampled sums, the others every slices-th token
+    for (int64_t g0 = 0; 64 * g0 < D; g0 += ROW_GROUPS) {
+        const int ng = (int)min((D + 63) / 64 - g0, (int64_t)ROW_GROUPS), slices = ROW_WAVES / ng - 1;
+        const int g = wave % ng, slice = wave / ng;
+        const int64_t c = min(64 * (g0 + g) + lane, D - 1);
+        if (slice == slices) {
+            float sum_abs, sum;
+            sampled_sums<DT>(a.x, base + c * a.sc, a.st * a.stride, ns, c < ncasc, sum_abs, sum);
+            s.sal[c] = sum_abs / (float)ns;
+            s.smean[c] = sum / (float)ns;
+        } else if (slice < slices) {
+            bool bad;
+            stats_slice<DT>(a.x, base + c * a.sc, a.st, slice, T, slices, part[wave].s1[lane], part[wave].s2[lane],
+                            part[wave].amax[lane], bad);
+            if (bad) s.bad = 1;
+        }
+        __syncthreads();
+        // one thread per channel of these groups
+        const int64_t co = 64 * g0 + tid;
+        if (wave < ng && co < D) {
+            double s1 = 0.0, s2 = 0.0;
+            float amax = 0.0f;
+            for (int k = 0; k < slices; ++k) {
+                const RowPart &p = part[wave + k * ng];
+                s1 = __dadd_rn(s1, p.s1[lane]);
+                s2 = __dadd_rn(s2, p.s2[lane]);
+                amax = fmaxf(amax, p.amax[lane]);
+            }
+            s.scale[co] = amax;
+            const IqErrRange r = iq_err_range(s1, s2, amax, s.smean[co], T);
+            s.err[co] = r.lo;
+            s.ehi[co] = r.hi;
+        }
+        __syncthreads();
+    }
+    row_select<DT, WIDE>(a, s, row, base);
+    if constexpr (WORDS)
+        quantize_words<DT, ROW_THREADS>(a, s.scale, s.is_src, s.src_of, *(RowTile<DT, ROW_THREADS> *)scratch, row, base, 0, T);
+    else
+        quantize_bytes<DT, ROW_THREADS>(a, s.scale, s.is_src, s.src_of, row, base, 0, T);
+}
+
+// ---- rows of more than LONG_ROW tokens
+//
+// Launch 1 leaves every partial result in the row's own payload bytes, which
+// nothing else holds until launch 3 writes them: per chunk of `chunk` tokens
+// the sums and largest magnitude of each channel, and the pieces of torch's
+// cascade sums of the sampled tokens.  A cascade adds 2^lp values from zero
+// into a level-0 sum, 2^lp of those into a level-1 sum and so on, so each
+// level-1 sum is its own piece (a workgroup's), and only the sums of pieces
+// are left for launch 2.  The columns past iq_cascade_columns(D) are four
+// interleaved cascades of a quarter of the samples each: a sequence is a
+// column, or one of those quarters.
+struct RowPlan {
+    int64_t chunk, nchunk;      // tokens per chunk, chunks
+    int64_t pieces;             // level-1 sums of the longest sequence, the unfinished one included
+    int64_t nseq;               // sequences
+    int64_t off_s2, off_amax, off_piece, bytes;
+};
+
+__host__ __device__ inline RowPlan row_plan(int64_t T, int64_t D, int64_t stride, int64_t chunk)
+{
+    RowPlan p;
+    const int64_t ns = (T + stride - 1) / stride, ncasc = iq_cascade_columns(D);
+    p.chunk = chunk;
+    p.nchunk = (T + chunk - 1) / chunk;
+    p.nseq = ncasc + 4 * (D - ncasc);
+    auto pieces = [](int64_t n) {
+        int lp = 0;
+        for (int64_t x = n > 1 ? n - 1 : 0; x; x >>= 1) ++lp;
+        lp = lp / 4 < 4 ? 4 : lp / 4;
+        return (n >> (2 * lp)) + 1;
+    };
+    const int64_t pc = ncasc > 0 ? pieces(ns) : 0, pr = ncasc < D ? pieces(ns / 4) : 0;
+    p.pieces = pc > pr ? pc : pr;
+    p.off_s2 = p.nchunk * D * 8;
+    p.off_amax = 2 * p.off_s2;
+    p.off_piece = p.off_amax + (p.nchunk * D * 4 + 7) / 8 * 8;
+    // piece k of sequence q: (sum of |x|, sum); slot `pieces`: the samples past the last whole level-0 sum
+    p.bytes = p.off_piece + (p.pieces + 1) * p.nseq * 8;
+    return p;
+}
+
+// The row's scratch: its payload bytes from the first 16-byte boundary on.
+__device__ __forceinline__ uint8_t *row_scratch(const K4Args &a, int64_t row)
+{
+    return (uint8_t *)(((uintptr_t)(a.payload + row * a.T * (a.D / 2)) + 15) & ~(uintptr_t)15);
+}
+
+struct RowSeq {
+    int64_t c, mul, add, n;     // channel, sample j * mul + add for j < n
+    int lp;
+    bool row_sum;
+};
+
+__device__ __forceinline__ RowSeq row_seq(int64_t q, int64_t ncasc, int64_t ns)
+{
+    RowSeq r;
+    r.row_sum = q >= ncasc;
+    r.c = r.row_sum ? ncasc + (q - ncasc) / 4 : q;
+    r.mul = r.row_sum ? 4 : 1;
+    r.add = r.row_sum ? (q - ncasc) % 4 : 0;
+    r.n = r.row_sum ? ns / 4 : ns;
+    r.lp = max(iq_ceil_log2(r.n) / 4, 4);
+    return r;
+}
+
+// Launch 1: grid (pieces, then chunks, rows).  WORDS: 16-byte loads.
+template <int DT, bool WORDS>
+__global__ __launch_bounds__(K4_THREADS) void k4_row_stats(K4Args a, RowPlan p)
+{
+    constexpr int WAVES = K4_THREADS / 64;
+    constexpr int MAXSUMS = 64;     // level-0 sums per level-1 sum: 2^lp, lp <= 6 for up to 2^27 samples
+    constexpr int WS = WORDS ? K4_THREADS * 4 : 1;
+    __shared__ union {
+        RowPart part[WAVES];
+        float2 sums[MAXSUMS][64];
+        struct {
+            double s1[WS], s2[WS];
+            float amax[WS];
+        } words;
+    } s;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t row = blockIdx.y, b = row / a.H, h = row % a.H;
+    const int64_t base = b * a.sb + h * a.sh, D = a.D;
+    uint8_t *const scratch = row_scratch(a, row);
+    // the pieces' workgroups first: they wait longest for their loads
+    const int64_t groups = (p.nseq + 63) / 64, npiece = p.pieces * groups;
+    if ((int64_t)blockIdx.x >= npiece) {
+        const int64_t k = blockIdx.x - npiece, t0 = k * p.chunk, t1 = min(t0 + p.chunk, a.T);
+        double *const out1 = (double *)scratch + k * D, *const out2 = (double *)(scratch + p.off_s2) + k * D;
+        float *const outm = (float *)(scratch + p.off_amax) + k * D;
+        if constexpr (WORDS) {
+            // lane (tt, j) = (tid / L, tid % L): channels 8 j .. of the tokens tt, tt + tps, ...
+            constexpr int EB = DT == IQ_F32 ? 4 : 2, NV = EB / 2, U = 8 / NV;
+            const int L = (int)D / 8, tps = K4_THREADS / L, tt = tid / L, j = tid - tt * L;
+            double s1[8], s2[8];
+            float amax[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                s1[e] = s2[e] = 0.0;
+                amax[e] = 0.0f;
+            }
+            bool bad = false;
+            if (tt < tps) {
+                const char *xb = (const char *)a.x + (base + 8 * j) * EB;
+                for (int64_t t = t0 + tt; t < t1; t += U * tps) {
+                    u32x4_t raw[U][NV];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const int64_t tc = t + u * tps < t1 ? t + u * tps : t;
+#pragma unroll
+                        for (int n = 0; n < NV; ++n) raw[u][n] = ((const u32x4_t *)(xb + tc * a.st * EB))[n];
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        if (t + u * tps >= t1) break;
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) {
+                            float v;
+                            if constexpr (EB == 4) v = __uint_as_float(raw[u][e / 4][e % 4]);
+                            else v = tile_f32<DT == IQ_F16>(e & 1 ? raw[u][0][e / 2] >> 16 : raw[u][0][e / 2] & 0xffffu);
+                            amax[e] = fmaxf(amax[e], fabsf(v));
+                            const double d = (double)v;
+                            s1[e] = __dadd_rn(s1[e], d);
+                            s2[e] = __builtin_fma(d, d, s2[e]);
+                        }
+                    }
+                }
+                // squares of finite floats sum to a finite double, any other value does not
+#pragma unroll
+                for (int e = 0; e < 8; ++e) bad |= !(s2[e] < (double)INFINITY);
+            }
+            if (bad) atomicOr(a.bad, 1);
+            // the tokens' sums meet in LDS, four channels of each lane at a time
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                const int W = (int)D / 2;            // channels of a half
+                if (tt < tps) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        // channel 8 j + 4 half + e at e L + j: neighbouring lanes on neighbouring banks
+                        s.words.s1[tt * W + e * L + j] = s1[4 * half + e];
+                        s.words.s2[tt * W + e * L + j] = s2[4 * half + e];
+                        s.words.amax[tt * W + e * L + j] = amax[4 * half + e];
+                    }
+                }
+                __syncthreads();
+                for (int c = tid; c < W; c += K4_THREADS) {
+                    double r1 = 0.0, r2 = 0.0;
+                    float rm = 0.0f;
+                    for (int i = 0; i < tps; ++i) {
+                        r1 = __dadd_rn(r1, s.words.s1[i * W + c]);
+                        r2 = __dadd_rn(r2, s.words.s2[i * W + c]);
+                        rm = fmaxf(rm, s.words.amax[i * W + c]);
+                    }
+                    const int e = c / L, ch = 8 * (c - e * L) + 4 * half + e;
+                    out1[ch] = r1;
+                    out2[ch] = r2;
+                    outm[ch] = rm;
+                }
+                __syncthreads();
+            }
+            return;
+        }
+        for (int64_t g0 = 0; 64 * g0 < D; g0 += WAVES) {
+            const int ng = (int)min((D + 63) / 64 - g0, (int64_t)WAVES), slices = WAVES / ng;
+            const int g = wave % ng, slice = wave / ng;
+            const int64_t c = min(64 * (g0 + g) + lane, D - 1);
+            if (slice < slices) {
+                bool bad;
+                stats_slice<DT>(a.x, base + c * a.sc, a.st, t0 + slice, t1, slices, s.part[wave].s1[lane],
+                                s.part[wave].s2[lane], s.part[wave].amax[lane], bad);
+                if (bad) atomicOr(a.bad, 1);
+            }
+            __syncthreads();
+            const int64_t co = 64 * g0 + tid;
+            if (wave < ng && co < D) {
+                double s1 = 0.0, s2 = 0.0;
+                float amax = 0.0f;
+                for (int i = 0; i < slices; ++i) {
+                    const RowPart &q = s.part[wave + i * ng];
+                    s1 = __dadd_rn(s1, q.s1[lane]);
+                    s2 = __dadd_rn(s2, q.s2[lane]);
+                    amax = fmaxf(amax, q.amax[lane]);
+                }
+                out1[co] = s1;
+                out2[co] = s2;
+                outm[co] = amax;
+            }
+            __syncthreads();
+        }
+        return;
+    }
+    // piece k of 64 sequences; the wavefronts share its level-0 sums
+    const int64_t k = blockIdx.x / groups, q0 = (blockIdx.x - k * groups) * 64;
+    const int64_t ns = (a.T + a.stride - 1) / a.stride, ncasc = iq_cascade_columns(D);
+    float2 *const piece = (float2 *)(scratch + p.off_piece);
+    const bool own = q0 + lane < p.nseq;
+    const int64_t q = own ? q0 + lane : p.nseq - 1;
+    const RowSeq r = row_seq(q, ncasc, ns);
+    const int64_t per = int64_t(1) << (2 * r.lp), first = k * per;
+    const int64_t left = r.n - first;                       // samples of this piece and the later ones
+    const int64_t nsum = left <= 0 ? 0 : min(left, per) >> r.lp;      // whole level-0 sums
+    const int64_t xb = base + r.c * a.sc, xs = a.st * a.stride;
+    auto level0 = [&](int64_t j0, int64_t j1) {              // samples j0 .. j1 - 1 added from zero
+        float2 acc = {0.0f, 0.0f};
+        for (int64_t jb = j0; jb < j1; jb += 16) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const int64_t jj = jb + u < j1 ? jb + u : j0;
+                v[u] = iq_load_f32(a.x, xb + (jj * r.mul + r.add) * xs, DT);
+            }
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                if (jb + u < j1) {
+                    acc.x = __fadd_rn(acc.x, fabsf(v[u]));
+                    acc.y = __fadd_rn(acc.y, v[u]);
+                }
+            }
+        }
+        return acc;
+    };
+    // the unfinished piece's samples past its last whole level-0 sum go to the last wavefront's lanes
+    const bool tail = left >= 0 && left < per;
+    if (r.lp == 4) {
+        // the usual length: the 16 samples of all four of a wavefront's sums in flight together
+        float v[4][16];
+        const int64_t sample = nsum > 0 ? r.mul * xs : 0;     // elements between a sequence's samples
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int64_t i = wave + WAVES * m, j0 = i < nsum ? first + 16 * i : 0;
+            int64_t at = xb + r.add * xs * (nsum > 0) + j0 * sample;
+#pragma unroll
+            for (int u = 0; u < 16; ++u, at += sample) v[m][u] = iq_load_f32(a.x, at, DT);
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            float2 acc = {0.0f, 0.0f};
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                acc.x = __fadd_rn(acc.x, fabsf(v[m][u]));
+                acc.y = __fadd_rn(acc.y, v[m][u]);
+            }
+            if (wave + WAVES * m < nsum) s.sums[wave + WAVES * m][lane] = acc;
+        }
+    } else {
+        for (int64_t i = wave; i < nsum; i += WAVES) s.sums[i][lane] = level0(first + (i << r.lp), first + ((i + 1) << r.lp));
+    }
+    if (wave == WAVES - 1 && own && tail) piece[p.pieces * p.nseq + q] = level0(first + (nsum << r.lp), r.n);
+    __syncthreads();
+    if (wave == 0 && own && left >= 0) {
+        float2 acc = {0.0f, 0.0f};
+        for (int64_t i = 0; i < nsum; ++i) {
+            acc.x = __fadd_rn(acc.x, s.sums[i][lane].x);
+            acc.y = __fadd_rn(acc.y, s.sums[i][lane].y);
+        }
+        piece[k * p.nseq + q] = acc;
+    }
+}
+
+// Launch 2: one workgroup per row adds the partial results and selects.
+template <int DT, bool WIDE>
+__global__ __launch_bounds__(ROW_THREADS) void k4_row_select(K4Args a, RowPlan p)
+{
+    __shared__ RowLds s;
+    __shared__ RowPart part[ROW_WAVES];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t row = blockIdx.x, b = row / a.H, h = row % a.H;
+    const int64_t base = b * a.sb + h * a.sh, D = a.D;
+    const uint8_t *const scratch = row_scratch(a, row);
+    const int64_t ns = (a.T + a.stride - 1) / a.stride, ncasc = iq_cascade_columns(D);
+    const float2 *const piece = (const float2 *)(scratch + p.off_piece);
+    if (tid == 0) s.bad = 0;
+    __syncthreads();
+    // the sampled sums of column c: one sequence, or four and their leftovers
+    auto cascade = [&](int64_t q) {
+        const RowSeq r = row_seq(q, ncasc, ns);
+        const int64_t whole = r.n >> (2 * r.lp);
+        float2 a2 = {0.0f, 0.0f}, a3 = {0.0f, 0.0f};
+        const float2 *pq = piece + q;
+        for (int64_t k0 = 0; k0 < whole; k0 += 8) {
+            float2 v[8];
+            const float2 *pk = pq;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                v[u] = *pk;
+                pk += k0 + u + 1 < whole ? p.nseq : 0;
+            }
+            pq = pk;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                if (k0 + u < whole) {
+                    a2.x = __fadd_rn(a2.x, v[u].x);
+                    a2.y = __fadd_rn(a2.y, v[u].y);
+                    if (((k0 + u + 1) & ((int64_t(1) << r.lp) - 1)) == 0) {
+                        a3.x = __fadd_rn(a3.x, a2.x);
+                        a3.y = __fadd_rn(a3.y, a2.y);
+                        a2 = {0.0f, 0.0f};
+                    }
+                }
+            }
+        }
+        const float2 a1 = piece[whole * p.nseq + q], a0 = piece[p.pieces * p.nseq + q];
+        return float2{__fadd_rn(__fadd_rn(__fadd_rn(a0.x, a1.x), a2.x), a3.x),
+                      __fadd_rn(__fadd_rn(__fadd_rn(a0.y, a1.y), a2.y), a3.y)};
+    };
+    // as in k4_encode_kernel: one wavefront of a channel group adds the
+    // sampled sums, the others the chunks
+    for (int64_t g0 = 0; 64 * g0 < D; g0 += ROW_GROUPS) {
+        const int ng = (int)min((D + 63) / 64 - g0, (int64_t)ROW_GROUPS), slices = ROW_WAVES / ng - 1;
+        const int g = wave % ng, slice = wave / ng;
+        const int64_t c = min(64 * (g0 + g) + lane, D - 1);
+        if (slice == slices) {
+            float2 sums;
+            if (c < ncasc) {
+                sums = cascade(c);
+            } else {
+                float2 quarter[4];
+                for (int k = 0; k < 4; ++k) quarter[k] = cascade(ncasc + 4 * (c - ncasc) + k);
+                for (int64_t r = ns / 4 * 4; r < ns; ++r) {
+                    const float v = iq_load_f32(a.x, base + c * a.sc + r * a.st * a.stride, DT);
+                    quarter[0].x = __fadd_rn(quarter[0].x, fabsf(v));
+                    quarter[0].y = __fadd_rn(quarter[0].y, v);
+                }
+                sums.x = __fadd_rn(__fadd_rn(__fadd_rn(quarter[0].x, quarter[1].x), quarter[2].x), quarter[3].x);
+                sums.y = __fadd_rn(__fadd_rn(__fadd_rn(quarter[0].y, quarter[1].y), quarter[2].y), quarter[3].y);
+            }
+            s.sal[c] = sums.x / (float)ns;
+            s.smean[c] = sums.y / (float)ns;
+        } else if (slice < slices) {
+            double s1 = 0.0, s2 = 0.0;
+            float amax = 0.0f;
+            // 32-bit indices: a uniform base and one add per load (few
+            // instructions: the launch's code is fetched by a handful of
+            // workgroups, once)
+            const double *p1 = (const double *)scratch, *p2 = (const double *)(scratch + p.off_s2);
+            const float *pm = (const float *)(scratch + p.off_amax);
+            const uint32_t n = (uint32_t)p.nchunk, step = (uint32_t)(slices * D), end = n * (uint32_t)D;
+            constexpr int U = 8;
+            for (uint32_t at = (uint32_t)(slice * D + c); at < end; at += U * step) {
+                double v1[U], v2[U];
+                float vm[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const uint32_t x = at + u * step < end ? at + u * step : at;
+                    v1[u] = p1[x];
+                    v2[u] = p2[x];
+                    vm[u] = pm[x];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const bool in = at + u * step < end;
+                    s1 = __dadd_rn(s1, in ? v1[u] : 0.0);
+                    s2 = __dadd_rn(s2, in ? v2[u] : 0.0);
+                    amax = fmaxf(amax, vm[u]);
+                }
+            }
+            part[wave].s1[lane] = s1;
+            part[wave].s2[lane] = s2;
+            part[wave].amax[lane] = amax;
+        }
+        __syncthreads();
+        const int64_t co = 64 * g0 + tid;
+        if (wave < ng && co < D) {
+            double s1 = 0.0, s2 = 0.0;
+            float amax = 0.0f;
+            for (int k = 0; k < slices; ++k) {
+                const RowPart &q = part[wave + k * ng];
+                s1 = __dadd_rn(s1, q.s1[lane]);
+                s2 = __dadd_rn(s2, q.s2[lane]);
+                amax = fmaxf(amax, q.amax[lane]);
+            }
+            s.scale[co] = amax;
+            const IqErrRange r = iq_err_range(s1, s2, amax, s.smean[co], a.T);
+            s.err[co] = r.lo;
+            s.ehi[co] = r.hi;
+            if (!iq_isfinite(amax) || s2 != s2) s.bad = 1;
+        }
+        __syncthreads();
+    }
+    row_select<DT, WIDE>(a, s, row, base);
+}
+
+// Launch 3: grid (tiles of q_tokens tokens, rows); a workgroup takes the row's
+// scales and descriptors from global memory.
+template <int DT, bool WORDS>
+__global__ __launch_bounds__(K4_THREADS) void k4_quantize_rows(K4Args a, int64_t q_tokens)
+{
+    __shared__ float s_scale[IQ_MAXD];
+    __shared__ int16_t s_src_of[IQ_MAXD];
+    __shared__ uint8_t s_is_src[IQ_MAXD];
+    __shared__ __attribute__((aligned(16))) RowTile<DT, WORDS ? K4_THREADS : 1> tile;
+    const int tid = threadIdx.x;
+    const int64_t row = blockIdx.y, b = row / a.H, h = row % a.H;
+    const int64_t base = b * a.sb + h * a.sh, D = a.D;
+    auto desc = [&](const void *p, int64_t i) -> int {
+        return a.desc_bytes == 1 ? ((const uint8_t *)p)[i]
+               : a.desc_bytes == 4 ? ((const int32_t *)p)[i] : (int)((const int64_t *)p)[i];
+    };
+    for (int64_t c = tid; c < D; c += K4_THREADS) {
+        s_scale[c] = a.scales[row * D + c];
+        s_is_src[c] = 0;
+        s_src_of[c] = -1;
+    }
+    __syncthreads();
+    for (int64_t i = tid; i < a.count; i += K4_THREADS) {
+        const int sc = desc(a.src, row * a.count + i), dn = desc(a.don, row * a.count + i);
+        s_is_src[sc] = 1;
+        s_src_of[dn] = (int16_t)sc;
+    }
+    __syncthreads();
+    const int64_t t0 = (int64_t)blockIdx.x * q_tokens, t1 = min(t0 + q_tokens, a.T);
+    if constexpr (WORDS) quantize_words<DT, K4_THREADS>(a, s_scale, s_is_src, s_src_of, tile, row, base, t0, t1);
+    else quantize_bytes<DT, K4_THREADS>(a, s_scale, s_is_src, s_src_of, row, base, t0, t1);
+}
+
+// ---------------------------------------------------------------------------
+// Tile encoder for the cache shapes: D = 128, 16-bit input, T <= 256 tokens,
+// channel-contiguous rows.  The block streams through LDS in 32-token chunks
+// (double-buffered, 16-byte loads, three chunks in flight while the current
+// one is consumed), twice:
+//   pass 1  waves 0-1: the fp64 Welford var_mean of channel tid (min_error
+//           only); delta / n uses a table of RN(1/n) and one remainder fma,
+//           which is the correctly rounded quotient for n <= 256 (sealed
+//           blocks: one fma with compile-time constants, see step_c);
+//           waves 2-3: sampled sums (torch cascade order), amax and
+//           finiteness as an integer max of the 16-bit magnitudes;
+//   then    donor selection by the whole workgroup (iq_select_tile128);
+//           the sequential donor picks run on one wavefront alone, and with a
+//           value row to encode (page mode, or VB = 2 / 4) the other three
+//           group-encode the values meanwhile (v_encode16, the same bits as
+//           v_encode_rows), reading them from HBM while it is otherwise idle;
+//   pass 2  every thread quantizes 8 channels of a token per step, writing
+//           4 payload bytes.
+// LDS stays under 40 KiB, so four blocks share a compute unit and their
+// latency-bound phases (the Welford chains, the donor picks) overlap.
+// Bit-identical to k4_encode_kernel.
+constexpr int TILE_D = 128;
+constexpr int TILE_T = 256;
+constexpr int CH = 32;                   // tokens per staged chunk
+constexpr int KPF = 1;                   // chunks in flight
+constexpr int XROW = TILE_D + 8;         // u16 per staged row: 68 dwords (16-byte aligned rows, distinct banks)
+// sealed blocks stream by direct global -> LDS loads into NBUF chunk buffers
+// (unpadded rows), NBUF - 1 chunks in flight while one is processed
+constexpr int NBUF_DMA = 4;
+
+// s_waitcnt vmcnt(2 * ahead) lgkmcnt(0), then s_barrier: this wave's loads
+// of every chunk but the `ahead` newest have landed in LDS and its LDS reads
+// are done; after the barrier the same holds for every wave.  Vector memory
+// operations retire in issue order, so at most 2 * ahead outstanding means
+// every older load is done; stores issued after a chunk's loads only make
+// the wait longer.  (A plain __syncthreads would wait for all loads in
+// flight.)
+__device__ __forceinline__ void wait_chunk_barrier(int ahead)
+{
+    switch (ahead) {
+    case 0: asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
+    case 1: asm volatile("s_waitcnt vmcnt(2) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
+    case 2: asm volatile("s_waitcnt vmcnt(4) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
+    default: asm volatile("s_waitcnt vmcnt(6) lgkmcnt(0)\n\ts_barrier" ::: "memory"); break;
+    }
+}
 
 // The V2 codes and group parameters of token t of head h in a page (value
 // lanes of 16 channels, vj = 0 .. 7, four lanes per 64-channel group).
@@ -1180,7 +1708,8 @@ __global__ __launch_bounds__(64) void reuse_map_kernel(SelectArgs a)
         if (a.err) s_err[c] = a.err[row * a.D + c];
     }
     __syncthreads();
-    iq_select_wave(s_sal, a.err ? s_err : nullptr, (int)a.D, (int)a.count, s_src, s_don, s_is_src, s_src_of);
+    if (a.D > 256) iq_select_wave<true>(s_sal, a.err ? s_err : nullptr, (int)a.D, (int)a.count, s_src, s_don, s_is_src, s_src_of);
+    else iq_select_wave<false>(s_sal, a.err ? s_err : nullptr, (int)a.D, (int)a.count, s_src, s_don, s_is_src, s_src_of);
     __syncthreads();
     for (int64_t i = threadIdx.x; i < a.count; i += 64) {
         a.src[row * a.count + i] = s_src[i];
@@ -1226,6 +1755,54 @@ bool tile_ok(const void *x, int dtype, const int64_t *s, int64_t T, int64_t D)
 
 }  // namespace
 
+namespace {
+
+// General rows: B * H rows of `a`.
+template <int DT>
+int launch_rows(const K4Args &a, int64_t B, hipStream_t st)
+{
+    const int64_t rows = B * a.H, T = a.T, D = a.D;
+    // quantize_words: 16-byte pieces of channel-contiguous rows, whole words out
+    constexpr int64_t EB = DT == IQ_F64 ? 8 : DT == IQ_F32 ? 4 : 2, VE = 16 / EB;
+    const bool words = DT != IQ_F64 && D % 8 == 0 && a.sc == 1 && a.st % VE == 0 && a.sh % VE == 0 && a.sb % VE == 0 &&
+                       ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.payload & 3) == 0;
+    // long rows (up to 2^24 tokens: the level-0 sums of a piece fit its LDS):
+    // chunks for about 1024 workgroups (eight rows of 32768 tokens: 63 us for
+    // the three launches, 68 with 512 and 83 with 2048), and the partial
+    // results in the row's payload bytes
+    constexpr int64_t MAXCH = 1024;
+    int64_t chunk = 64;
+    while (chunk < 1024 && rows * ((T + chunk - 1) / chunk) > MAXCH) chunk *= 2;
+    const RowPlan p = row_plan(T, D, a.stride, chunk);
+    if (T > LONG_ROW && T <= (int64_t(1) << 24) && rows <= 65535 && p.bytes + 15 <= T * (D / 2)) {
+        const dim3 parts((unsigned)(p.nchunk + p.pieces * ((p.nseq + 63) / 64)), (unsigned)rows);
+        const dim3 tiles((unsigned)p.nchunk, (unsigned)rows);
+        if constexpr (DT != IQ_F64) {
+            if (words) hipLaunchKernelGGL((k4_row_stats<DT, true>), parts, dim3(K4_THREADS), 0, st, a, p);
+        }
+        if (!words) hipLaunchKernelGGL((k4_row_stats<DT, false>), parts, dim3(K4_THREADS), 0, st, a, p);
+        if (D > 256) hipLaunchKernelGGL((k4_row_select<DT, true>), dim3((unsigned)rows), dim3(ROW_THREADS), 0, st, a, p);
+        else hipLaunchKernelGGL((k4_row_select<DT, false>), dim3((unsigned)rows), dim3(ROW_THREADS), 0, st, a, p);
+        if constexpr (DT != IQ_F64) {
+            if (words) hipLaunchKernelGGL((k4_quantize_rows<DT, true>), tiles, dim3(K4_THREADS), 0, st, a, p.chunk);
+        }
+        if (!words) hipLaunchKernelGGL((k4_quantize_rows<DT, false>), tiles, dim3(K4_THREADS), 0, st, a, p.chunk);
+        IQ_CHECK_LAUNCH("k4_row_stats, k4_row_select, k4_quantize_rows");
+        return IQ_OK;
+    }
+    const dim3 grid((unsigned)rows), block(ROW_THREADS);
+    if constexpr (DT != IQ_F64) {
+        if (words && D > 256) hipLaunchKernelGGL((k4_encode_kernel<DT, true, true>), grid, block, 0, st, a);
+        else if (words) hipLaunchKernelGGL((k4_encode_kernel<DT, true, false>), grid, block, 0, st, a);
+    }
+    if (!words && D > 256) hipLaunchKernelGGL((k4_encode_kernel<DT, false, true>), grid, block, 0, st, a);
+    else if (!words) hipLaunchKernelGGL((k4_encode_kernel<DT, false, false>), grid, block, 0, st, a);
+    IQ_CHECK_LAUNCH("k4_encode_kernel");
+    return IQ_OK;
+}
+
+}  // namespace
+
 extern "C" int iq_k4_quantize(const void *x, int x_dtype, const int64_t *x_strides, int64_t B, int64_t H,
                               int64_t T, int64_t D, int64_t count, int64_t sample_stride, int min_error,
                               uint8_t *payload, float *scales, void *src, void *don, int desc_bytes,
@@ -1256,17 +1833,13 @@ extern "C" int iq_k4_quantize(const void *x, int x_dtype, const int64_t *x_strid
         IQ_CHECK_LAUNCH("k4_encode_tile");
         return IQ_OK;
     }
-    // long rows: the per-row statistics on one workgroup each, the payload
-    // spread over token tiles
-    a.split = T > 4 * Q_TOKENS && B * H <= 65535 ? 1 : 0;
-    hipLaunchKernelGGL(k4_encode_kernel, dim3((unsigned)(B * H)), dim3(K4_THREADS), 0, (hipStream_t)stream, a);
-    IQ_CHECK_LAUNCH("k4_encode_kernel");
-    if (a.split) {
-        hipLaunchKernelGGL(k4_quantize_generic, dim3((unsigned)((T + Q_TOKENS - 1) / Q_TOKENS), (unsigned)(B * H)),
-                           dim3(K4_THREADS), 0, (hipStream_t)stream, a);
-        IQ_CHECK_LAUNCH("k4_quantize_generic");
+    const hipStream_t st = (hipStream_t)stream;
+    switch (x_dtype) {
+    case IQ_BF16: return launch_rows<IQ_BF16>(a, B, st);
+    case IQ_F16: return launch_rows<IQ_F16>(a, B, st);
+    case IQ_F64: return launch_rows<IQ_F64>(a, B, st);
+    default: return launch_rows<IQ_F32>(a, B, st);
     }
-    return IQ_OK;
 }
 
 namespace {

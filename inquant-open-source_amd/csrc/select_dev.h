@@ -389,13 +389,18 @@ __device__ __forceinline__ void iq_select_wave128(const float *sal, const float 
     iq_pick_donors128(sal, sel0, sel1, av0, av1, count, src_out, don_out, is_src, src_of, list);
 }
 
+// WIDE: D > 256.
+template <bool WIDE>
 __device__ __forceinline__ void iq_select_wave(const float *sal, const float *err, int D, int count,
                                                int16_t *src_out, int16_t *don_out, uint8_t *is_src,
                                                int16_t *src_of)
 {
-    if (D <= 64) iq_select_wave_t<1>(sal, err, D, count, src_out, don_out, is_src, src_of);
-    else if (D <= 128) iq_select_wave_t<2>(sal, err, D, count, src_out, don_out, is_src, src_of);
-    else if (D <= 256) iq_select_wave_t<4>(sal, err, D, count, src_out, don_out, is_src, src_of);
-    else if (D <= 512) iq_select_wave_t<8>(sal, err, D, count, src_out, don_out, is_src, src_of);
-    else iq_select_wave_t<16>(sal, err, D, count, src_out, don_out, is_src, src_of);
+    if constexpr (WIDE) {
+        if (D <= 512) iq_select_wave_t<8>(sal, err, D, count, src_out, don_out, is_src, src_of);
+        else iq_select_wave_t<16>(sal, err, D, count, src_out, don_out, is_src, src_of);
+    } else {
+        if (D <= 64) iq_select_wave_t<1>(sal, err, D, count, src_out, don_out, is_src, src_of);
+        else if (D <= 128) iq_select_wave_t<2>(sal, err, D, count, src_out, don_out, is_src, src_of);
+        else iq_select_wave_t<4>(sal, err, D, count, src_out, don_out, is_src, src_of);
+    }
 }

@@ -1,0 +1,101 @@
+"""General-row K4 encoder: rows of one workgroup, rows spread over the chip,
+and the certified donor errors both take from order-free sums
+(csrc/k4_stats_dev.h)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle
+import synth
+
+F = np.float32
+
+
+def _err_range(x, smean):
+    """iq_err_range of the rows x [n, channels] (float32)."""
+    n = x.shape[0]
+    d = x.astype(np.float64)
+    s1, s2 = d.sum(0), (d * d).sum(0)
+    a = np.abs(x).max(0).astype(np.float64)
+    inv = 1.0 / n
+    mean = s1 * inv
+    var = s2 * inv - mean * mean
+    e, h = a * ((2 * n + 32) * 2.0 ** -53), a * a * ((n + 16) * 2.0 ** -49)
+    with np.errstate(over="ignore", invalid="ignore"):
+        vlo, vhi = np.maximum(var - h, 0).astype(F), np.maximum(var + h, 0).astype(F)
+        da, db = (mean - e).astype(F) - smean, (mean + e).astype(F) - smean
+        qa, qb = da * da, db * db
+        return vlo + np.where((da < 0) & (db > 0), F(0), np.minimum(qa, qb)), vhi + np.maximum(qa, qb)
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 17, 256, 4096, 32768])
+def test_error_range_encloses_the_sequential_pass(n):
+    rng = np.random.default_rng(n)
+    c = 48
+    base = rng.standard_normal((n, c))
+    rows = [base, base * 1e-3 + 5.0, base * 2.0 ** rng.integers(-60, 60, c), np.exp(6 * base), base * 1e-30,
+            np.full((n, c), 1.0 / 3.0) + 1e-6 * (np.arange(n) % 2)[:, None], np.zeros((n, c)),
+            np.where(np.arange(n)[:, None] == n - 1, 1e4, base), np.sort(base, 0), 1e18 * base, 3e38 * np.tanh(base)]
+    for x in rows:
+        for y in (x.astype(F), synth.bf16_round(x.astype(F))):
+            with np.errstate(over="ignore", invalid="ignore"):
+                sal, smean, err, amax = oracle.k4_stats(y, 8, True)
+                lo, hi = _err_range(y, smean)
+                ok = np.isfinite(smean)
+                assert (lo <= hi)[ok].all()
+                assert ((lo <= err) & (err <= hi))[ok].all()
+
+
+def _check(x, stride, frac, policy):
+    from inquant.codec import CodecConfig, quantize
+    ref = oracle.k4_quantize(np.ascontiguousarray(x.float().cpu().numpy()), stride, frac, policy)
+    got = quantize(x, CodecConfig(sample_stride=stride, salient_fraction=frac, donor_policy=policy))
+    for field in ("payload", "scales", "salient_channels", "donor_channels", "padding"):
+        a, b = got.tensors[field].cpu().numpy(), ref[field]
+        np.testing.assert_array_equal(a.astype(b.dtype).view(np.uint8), b.view(np.uint8), err_msg=field)
+
+
+# around the length where a row leaves its workgroup (256), the chunk and piece lengths (64 tokens, 256 samples), and
+# the head sizes of one, several and partly filled channel groups and of torch's two summation orders
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,T,stride,policy,frac,dtype", [
+    (64, 256, 8, "min_error", 0.125, torch.float16), (64, 256, 8, "min_error", 0.125, torch.float32),
+    (64, 257, 8, "min_error", 0.125, torch.float16), (96, 511, 1, "min_error", 0.25, torch.bfloat16),
+    (96, 2049, 1, "min_error", 0.5, torch.float32), (128, 513, 1, "min_error", 0.125, torch.bfloat16),
+    (128, 4096, 16, "neighbors", 0.125, torch.bfloat16), (128, 4095, 2, "min_error", 0.125, torch.float32),
+    (128, 70000, 1, "min_error", 0.125, torch.bfloat16), (130, 1025, 3, "min_error", 0.125, torch.float16),
+    (2, 4100, 1, "min_error", 0.5, torch.float32), (6, 700, 1, "min_error", 0.33, torch.float32),
+    (258, 640, 5, "min_error", 0.5, torch.bfloat16), (1024, 600, 8, "min_error", 0.125, torch.float32),
+    (1024, 65, 8, "min_error", 0.5, torch.bfloat16), (72, 2000, 2, "min_error", 0.125, torch.float16),
+    (40, 1111, 999999, "min_error", 0.125, torch.float64), (32, 600, 8, "min_error", 0.0, torch.bfloat16)])
+def test_rows_match_the_oracle(D, T, stride, policy, frac, dtype):
+    x = synth.normal(D * 77 + T, (1, 2, T, D)) * np.exp(synth.normal(T, (1, 2, 1, D)))
+    x[..., 1:3] *= 25
+    _check(torch.from_numpy(x).cuda().to(torch.float64).to(dtype), stride, frac, policy)
+
+
+# channels whose errors tie or differ by less than the order-free sums resolve: the row takes the sequential pass
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [40, 300, 1500])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_rows_with_tied_errors(T, dtype):
+    x = synth.normal(T, (1, 3, T, 64))
+    x[0, 0, :, 8:] = x[0, 0, :, 8:9]                    # 56 equal channels
+    x[0, 1, :, 20:50] = np.arange(20, 50) / 7.0         # 30 constant channels
+    x[0, 2, :, 4:60] = x[0, 2, ::-1, 4:5]               # equal channels in another token order
+    x[0, 2, :, 5:60:2] = x[0, 2, ::-1, 5:60:2]
+    _check(torch.from_numpy(np.ascontiguousarray(x)).cuda().to(dtype), 8, 0.25, "min_error")
+    _check(torch.zeros((1, 1, T, 64), dtype=dtype, device="cuda"), 8, 0.25, "min_error")
+
+
+# layouts that the 16-byte pieces of quantize_words cannot take, and those they can
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [48, 700])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_row_layouts(T, dtype):
+    x = torch.from_numpy(synth.normal(5 * T, (2, T + 1, 3, 80))).cuda().to(dtype)
+    for view in (x[:, 1:].transpose(1, 2), x[:, :T, :, 8:72].transpose(1, 2), x[:, :T, :, 3:67].transpose(1, 2),
+                 x[:, :T].permute(0, 2, 1, 3)[..., ::2], x[:1, :T].transpose(1, 2).expand(3, -1, -1, -1),
+                 x[:, :T].transpose(1, 2).transpose(0, 1)):
+        _check(view, 8, 0.125, "min_error")
+
