@@ -99,3 +99,30 @@ def test_row_layouts(T, dtype):
                  x[:, :T].transpose(1, 2).transpose(0, 1)):
         _check(view, 8, 0.125, "min_error")
 
+
+# the pool picks (at most 16 sources, as many donors) and the bit-scan picks past them: runs, ties, the first and the
+# last channel
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [2, 34, 64, 128, 130, 256, 1024])
+@pytest.mark.parametrize("count", [1, 15, 16, 17])
+def test_pool_picks(D, count):
+    from inquant.codec import _reuse_map
+    if 2 * count > D:
+        pytest.skip("more sources than donors")
+    rows = []
+    for i in range(24):
+        sal, err = np.abs(synth.normal(i, (D,))), np.abs(synth.normal(100 + i, (D,)))
+        if i % 3 == 0:
+            sal, err = np.round(2 * sal), np.round(2 * err)             # ties
+        if i % 4 == 1:
+            sal[(i * 5) % D:(i * 5) % D + 6] += 9                       # a run of sources
+            sal[-2:] += 9
+        if i % 4 == 2:
+            sal[:3] += 9
+            err[:] = np.sort(err)                                       # the pool beside them
+        rows.append((sal, err))
+    sal, err = (np.stack([r[k] for r in rows]).astype(F) for k in (0, 1))
+    want = oracle.reuse_map(sal, count, err)
+    got = _reuse_map(torch.from_numpy(sal).cuda(), count, torch.from_numpy(err).cuda())
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(a.cpu().numpy(), b)
