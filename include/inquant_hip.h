@@ -22,6 +22,8 @@
  *   iq_reuse_map        src/inquant/triton_selection.py:46-60 reuse_map(),
  *                       src/inquant/codec.py:137-178         _reuse_map()
  *   iq_k4_dequantize    src/inquant/codec.py:112-134         PackedTensor.dequantize()
+ *   iq_k4_dequantize_into, iq_v_dequantize_into, iq_copy_rows
+ *                       src/inquant/cache.py:328-345         InQuantCache materialize
  *   iq_v_quantize       src/inquant/value_codec.py:51-72     quantize_values()
  *   iq_v_dequantize     src/inquant/value_codec.py:38-48     PackedValues.dequantize()
  *   iq_kv_quantize      src/inquant/cache.py:288-295 (the paired key / value block
@@ -97,6 +99,15 @@ int iq_k4_dequantize(const uint8_t *payload, const float *scales, const void *sr
                      int64_t count, void *out, int out_dtype, void *stream);
 
 /*
+ * The same for rows (b, h) of a batch [B, H]: token t of row (b, h) goes to
+ * out + b out_sb + h out_sh + t D (element strides), as a cache's blocks do
+ * into its dense history (cache.py:328-345).
+ */
+int iq_k4_dequantize_into(const uint8_t *payload, const float *scales, const void *src, const void *don,
+                          int desc_bytes, const float *padding, int64_t B, int64_t H, int64_t T, int64_t D,
+                          int64_t count, void *out, int out_dtype, int64_t out_sb, int64_t out_sh, void *stream);
+
+/*
  * Group-wise affine value encode of x[B, H, T, D] (strides x_strides[4]):
  * bits in {2, 4}, group in {32, 64, 128}, D % group == 0.  Outputs
  * payload u8 [B,H,T,D*bits/8]; scales/offsets f16 bits [B,H,T,D/group].
@@ -141,6 +152,11 @@ int iq_k4_quantize_kv(const void *keys, const void *values, int dtype, const int
 /* Value decode: out [rows, D] of out_dtype (rows = B*H*T); value_codec.py:38-48. */
 int iq_v_dequantize(const uint8_t *payload, const uint16_t *scales, const uint16_t *offsets,
                     int64_t rows, int64_t D, int bits, int group, void *out, int out_dtype, void *stream);
+
+/* The same with the output placed as by iq_k4_dequantize_into. */
+int iq_v_dequantize_into(const uint8_t *payload, const uint16_t *scales, const uint16_t *offsets, int64_t B, int64_t H,
+                         int64_t T, int64_t D, int bits, int group, void *out, int out_dtype, int64_t out_sb,
+                         int64_t out_sh, void *stream);
 
 /*
  * One sealed block's device addresses, as recorded in the decode state's
@@ -408,6 +424,21 @@ typedef struct iq_tail_desc {
 
 int iq_tail_append_row(const iq_tail_desc *desc, const void *k, const void *v, int64_t slot, int64_t shift_src,
                        int64_t shift_count, const void *positions, int64_t expected, void *stream);
+
+/*
+ * Copies of [H, tokens] rows of row_bytes bytes, up to IQ_COPY_SEGMENTS
+ * segments in one launch (byte strides of heads and tokens; the segments'
+ * sources and destinations must not overlap): a cache's dense rows
+ * (cache.py:256-259,328-345).
+ */
+#define IQ_COPY_SEGMENTS 8
+
+typedef struct iq_copy_segment {
+    uint64_t src, dst;
+    int64_t src_h, src_t, dst_h, dst_t, tokens;
+} iq_copy_segment;
+
+int iq_copy_rows(const iq_copy_segment *segments, int64_t n, int64_t H, int64_t row_bytes, void *stream);
 
 #ifdef __cplusplus
 }

@@ -56,6 +56,29 @@ __global__ __launch_bounds__(64) void tail_append_kernel(TailArgs a)
     }
 }
 
+// Rows of up to IQ_COPY_SEGMENTS segments, 16 lanes a row, 16 rows a
+// workgroup: what a cache's first tokens, tail and new tokens need at once.
+struct CopyArgs {
+    iq_copy_segment seg[IQ_COPY_SEGMENTS];
+    int64_t first[IQ_COPY_SEGMENTS + 1];        // rows before segment i
+    int n;
+    int64_t H, row_units;
+};
+
+template <typename U>
+__global__ __launch_bounds__(256) void copy_rows_kernel(CopyArgs a)
+{
+    const int64_t r = (int64_t)blockIdx.x * 16 + (threadIdx.x >> 4);
+    if (r >= a.first[a.n]) return;
+    int k = 0;
+    while (r >= a.first[k + 1]) ++k;
+    const iq_copy_segment g = a.seg[k];
+    const int64_t i = r - a.first[k], t = i / a.H, h = i - t * a.H;
+    const U *src = (const U *)((const char *)g.src + h * g.src_h + t * g.src_t);
+    U *dst = (U *)((char *)g.dst + h * g.dst_h + t * g.dst_t);
+    for (int64_t u = threadIdx.x & 15; u < a.row_units; u += 16) dst[u] = src[u];
+}
+
 }  // namespace
 
 extern "C" int iq_tail_append(const void *k, const void *v, int64_t k_sh, int64_t k_st, int64_t v_sh, int64_t v_st,
@@ -121,4 +144,45 @@ extern "C" int iq_tail_append_row(const iq_tail_desc *d, const void *k, const vo
     return iq_tail_append(k, v, d->k_sh, d->k_st, d->v_sh, d->v_st, d->heads, 1, d->dim, d->elem_bytes,
                           (void *)d->buf, d->buf_kv, d->buf_h, d->buf_t, d->capacity, slot, shift_src, shift_count,
                           positions, d->pos_bytes, expected, (int *)d->flag, stream);
+}
+
+extern "C" int iq_copy_rows(const iq_copy_segment *segments, int64_t n, int64_t H, int64_t row_bytes, void *stream)
+{
+    IQ_CHECK_ARG(n >= 0 && n <= IQ_COPY_SEGMENTS && (n == 0 || segments), "iq_copy_rows: at most %d segments",
+                 IQ_COPY_SEGMENTS);
+    IQ_CHECK_ARG(H >= 1 && row_bytes >= 1, "iq_copy_rows: bad shape");
+    CopyArgs a{};
+    a.H = H;
+    int64_t bits = row_bytes, rows = 0;
+    for (int64_t i = 0; i < n; ++i) {
+        const iq_copy_segment &g = segments[i];
+        IQ_CHECK_ARG(g.tokens >= 0, "iq_copy_rows: bad shape");
+        if (g.tokens == 0) continue;
+        IQ_CHECK_ARG(g.src && g.dst, "iq_copy_rows: null pointer");
+        a.seg[a.n] = g;
+        a.first[a.n++] = rows;
+        rows += g.tokens * H;
+        bits |= (int64_t)g.src | (int64_t)g.dst | g.src_h | g.src_t | g.dst_h | g.dst_t;
+    }
+    a.first[a.n] = rows;
+    if (rows == 0) return IQ_OK;
+    IQ_CHECK_ARG((rows + 15) / 16 <= 0x7fffffffLL, "iq_copy_rows: too many rows");
+    const dim3 grid((unsigned)((rows + 15) / 16)), block(256);
+    const hipStream_t s = (hipStream_t)stream;
+    // the widest unit that every address, stride and the row length allow
+    if (bits % 16 == 0) {
+        a.row_units = row_bytes / 16;
+        hipLaunchKernelGGL(copy_rows_kernel<uint4>, grid, block, 0, s, a);
+    } else if (bits % 4 == 0) {
+        a.row_units = row_bytes / 4;
+        hipLaunchKernelGGL(copy_rows_kernel<uint32_t>, grid, block, 0, s, a);
+    } else if (bits % 2 == 0) {
+        a.row_units = row_bytes / 2;
+        hipLaunchKernelGGL(copy_rows_kernel<uint16_t>, grid, block, 0, s, a);
+    } else {
+        a.row_units = row_bytes;
+        hipLaunchKernelGGL(copy_rows_kernel<uint8_t>, grid, block, 0, s, a);
+    }
+    IQ_CHECK_LAUNCH("copy_rows_kernel");
+    return IQ_OK;
 }

@@ -210,26 +210,29 @@ bool v_rows_dispatch_gl(int GL, int PR, dim3 grid, hipStream_t st, const VRowArg
     }
 }
 
+// rows of D channels: row (b, h) holds T tokens, token t of it goes to out +
+// b osb + h osh + t D (element strides; H heads)
 struct VDecArgs {
     const uint8_t *payload;
     const uint16_t *scales, *offsets;
-    int64_t rows, D;
+    int64_t H, T, D;
     int bits, group;
     void *out;
     int out_dt;
+    int64_t osb, osh;
 };
 
 __global__ __launch_bounds__(V_THREADS) void v_decode_kernel(VDecArgs a)
 {
     const int64_t i = (int64_t)blockIdx.x * V_THREADS + threadIdx.x;
-    if (i >= a.rows * a.D) return;
-    const int64_t r = i / a.D, c = i - r * a.D;
+    if (i >= a.T * a.D) return;
+    const int64_t row = blockIdx.y, t = i / a.D, c = i - t * a.D, r = row * a.T + t;
     const int per_byte = 8 / a.bits;
     const int code = (a.payload[r * (a.D / per_byte) + c / per_byte] >> ((c % per_byte) * a.bits)) &
                      ((1 << a.bits) - 1);
     const int64_t p = r * (a.D / a.group) + c / a.group;
     const float v = __fadd_rn(__fmul_rn((float)code, iq_f16_to_f32(a.scales[p])), iq_f16_to_f32(a.offsets[p]));
-    iq_store_as(a.out, i, v, a.out_dt);
+    iq_store_as(a.out, row / a.H * a.osb + row % a.H * a.osh + i, v, a.out_dt);
 }
 
 struct KDecArgs {
@@ -241,7 +244,14 @@ struct KDecArgs {
     int64_t rows, T, D, count;
     void *out;
     int out_dt;
+    int64_t H, osb, osh;        // row (b, h) goes to out + b osb + h osh
 };
+
+__device__ __forceinline__ int64_t out_row(const KDecArgs &a, int64_t row)
+{
+    const uint32_t b = (uint32_t)row / (uint32_t)a.H;       // rows <= 2^31
+    return b * a.osb + ((uint32_t)row - b * (uint32_t)a.H) * a.osh;
+}
 
 __device__ __forceinline__ int load_desc(const void *p, int64_t i, int bytes)
 {
@@ -278,7 +288,7 @@ __global__ __launch_bounds__(V_THREADS) void k4_decode_kernel(KDecArgs a)
         } else {
             v = __fmul_rn((float)(slot - 8), a.scales[row * a.D + c]);
         }
-        iq_store_as(a.out, rt * a.D + c, v, a.out_dt);
+        iq_store_as(a.out, out_row(a, row) + (rt - row * a.T) * a.D + c, v, a.out_dt);
     }
 }
 
@@ -298,23 +308,27 @@ __device__ __forceinline__ uint32_t pack_pair(float x, float y)
     }
 }
 
-// Rows of 128 channels, 16-byte aligned output rows.  Thread (row, j)
-// decodes channels 16 j .. 16 j + 15 of one row: BITS / 2 payload words and
-// its group's f16 scale and offset, then writes 16 values with 16-byte
-// stores.  Same arithmetic as v_decode_kernel.
-template <int BITS, int OUT>
+// 16-byte aligned output rows.  Thread (token, j) decodes channels 16 j ..
+// 16 j + 15 of a token: BITS / 2 payload words and its group's f16 scale and
+// offset, then writes 16 values with 16-byte stores.  Same arithmetic as
+// v_decode_kernel.  L: D / 16, or 0 for one read from the arguments.  Bound by
+// its writes: the 2-bit values of 32512 tokens x 8 heads of 128 channels into
+// their place of a dense history in 19 us (76 MB, 15 us at the rate of a
+// copy); dequantized first and copied there it was 17.8 us and a strided copy
+// of the 67 MB.
+template <int BITS, int OUT, int L>
 __global__ __launch_bounds__(V_THREADS) void v_decode_rows(VDecArgs a)
 {
-    const int64_t u = (int64_t)blockIdx.x * V_THREADS + threadIdx.x;
-    const int64_t r = u >> 3;
-    const int j = (int)(u & 7);
-    if (r >= a.rows) return;
-    constexpr int PB = 128 * BITS / 8;                      // payload bytes per row
-    const int64_t p = r * (128 / a.group) + (16 * j) / a.group;
+    const uint32_t u = blockIdx.x * V_THREADS + threadIdx.x, l = L ? L : (uint32_t)a.D / 16;
+    const uint32_t t = u / l, j = u - t * l;
+    if (t >= (uint32_t)a.T) return;
+    const uint32_t row = blockIdx.y, b = row / (uint32_t)a.H;
+    const int64_t r = row * a.T + t, at = b * a.osb + (row - b * (uint32_t)a.H) * a.osh + (int64_t)t * a.D + 16 * j;
+    const int64_t p = r * ((uint32_t)a.D / (uint32_t)a.group) + (16 * j) / (uint32_t)a.group;
     const float sc = iq_f16_to_f32(a.scales[p]), off = iq_f16_to_f32(a.offsets[p]);
     uint64_t w;                                             // channel 16 j + e at bits BITS * e
-    if constexpr (BITS == 2) w = *(const uint32_t *)(a.payload + r * PB + 4 * j);
-    else w = *(const uint64_t *)(a.payload + r * PB + 8 * j);
+    if constexpr (BITS == 2) w = ((const uint32_t *)a.payload)[r * l + j];
+    else w = ((const uint64_t *)a.payload)[r * l + j];
     float v[16];
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
@@ -322,14 +336,14 @@ __global__ __launch_bounds__(V_THREADS) void v_decode_rows(VDecArgs a)
         v[e] = __fadd_rn(__fmul_rn((float)code, sc), off);
     }
     if constexpr (OUT == IQ_F32) {
-        float4 *o = (float4 *)((float *)a.out + r * 128 + 16 * j);
+        float4 *o = (float4 *)((float *)a.out + at);
 #pragma unroll
         for (int k = 0; k < 4; ++k) o[k] = float4{v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]};
     } else {
         uint32_t h[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) h[k] = pack_pair<OUT>(v[2 * k], v[2 * k + 1]);
-        u32x4_nt *o = (u32x4_nt *)((uint16_t *)a.out + r * 128 + 16 * j);
+        u32x4_nt *o = (u32x4_nt *)((uint16_t *)a.out + at);
         __builtin_nontemporal_store(u32x4_nt{h[0], h[1], h[2], h[3]}, o);
         __builtin_nontemporal_store(u32x4_nt{h[4], h[5], h[6], h[7]}, o + 1);
     }
@@ -362,6 +376,7 @@ __global__ __launch_bounds__(V_THREADS) void k4_decode_rows(KDecArgs a)
         const int64_t rt = row * a.T + (t < a.T ? t : a.T - 1);   // every lane loads (the shuffles need all)
         words[i] = *(const uint32_t *)(a.payload + rt * 64 + 4 * j);
     }
+    const int64_t obase = out_row(a, row);
     if (tid < 128) {
         s_scale[tid] = a.scales[row * 128 + tid];
         s_role[tid] = -1;
@@ -405,7 +420,7 @@ __global__ __launch_bounds__(V_THREADS) void k4_decode_rows(KDecArgs a)
     for (int i = 0; i < KD_ITER; ++i) {
         const int64_t t = t_first + i * (V_THREADS / 16);
         const bool live = t < a.T;
-        const int64_t rt = row * a.T + (live ? t : a.T - 1);
+        const int64_t at = obase + t * 128 + 8 * j;
         const uint32_t w = words[i];
         uint32_t x[8];
 #pragma unroll
@@ -421,14 +436,93 @@ __global__ __launch_bounds__(V_THREADS) void k4_decode_rows(KDecArgs a)
         }
         if (!live) continue;
         if constexpr (OUT == IQ_F32) {
-            float4 *o = (float4 *)((float *)a.out + rt * 128 + 8 * j);
+            float4 *o = (float4 *)((float *)a.out + at);
             o[0] = float4{v[0], v[1], v[2], v[3]};
             o[1] = float4{v[4], v[5], v[6], v[7]};
         } else {
             uint32_t h[4];
 #pragma unroll
             for (int k = 0; k < 4; ++k) h[k] = pack_pair<OUT>(v[2 * k], v[2 * k + 1]);
-            __builtin_nontemporal_store(u32x4_nt{h[0], h[1], h[2], h[3]}, (u32x4_nt *)((uint16_t *)a.out + rt * 128 + 8 * j));
+            __builtin_nontemporal_store(u32x4_nt{h[0], h[1], h[2], h[3]}, (u32x4_nt *)((uint16_t *)a.out + at));
+        }
+    }
+}
+
+// Any head size that is a multiple of 8, any descriptor width, 16-byte aligned
+// output rows.  Grid (tiles of KW_STEPS steps, rows): a workgroup takes 256 /
+// (D / 8) tokens a step, thread (tt, j) channels 8 j .. 8 j + 7 of one; the
+// step's words meet in LDS, where a source finds its donor's nibble.  The slot
+// arithmetic of k4_decode_rows.  (One workgroup per token, with the role map
+// rebuilt in each, took 150 us for eight rows of 32768 bf16 tokens x 64 channels;
+// this takes 10.7: 42 MB, 8.2 us at the rate of a copy.)
+constexpr int KW_STEPS = 4;
+
+template <int OUT>
+__global__ __launch_bounds__(V_THREADS) void k4_decode_words(KDecArgs a)
+{
+    __shared__ float s_scale[1024], s_pad[512];
+    __shared__ int16_t s_role[1024];
+    __shared__ uint32_t s_word[KW_STEPS][V_THREADS];
+    const int tid = threadIdx.x, D = (int)a.D, L = D / 8, tps = V_THREADS / L, tt = tid / L, j = tid - tt * L;
+    const int64_t row = blockIdx.y, t0 = (int64_t)blockIdx.x * (KW_STEPS * tps) + tt;
+    const uint32_t *const words = (const uint32_t *)a.payload + row * a.T * L + j;
+#pragma unroll
+    for (int i = 0; i < KW_STEPS; ++i) {
+        const int64_t t = t0 + i * tps;
+        s_word[i][tid] = words[(t < a.T ? t : a.T - 1) * L];
+    }
+    for (int c = tid; c < D; c += V_THREADS) {
+        s_scale[c] = a.scales[row * D + c];
+        s_role[c] = -1;
+    }
+    __syncthreads();
+    for (int i = tid; i < (int)a.count; i += V_THREADS) {
+        const int sch = load_desc(a.src, row * a.count + i, a.desc_bytes);
+        const int dch = load_desc(a.don, row * a.count + i, a.desc_bytes);
+        if ((uint32_t)sch < (uint32_t)D && (uint32_t)dch < (uint32_t)D) {
+            s_role[sch] = (int16_t)dch;
+            s_role[dch] = (int16_t)(-2 - i);
+        }
+        s_pad[i] = a.padding[row * a.count + i];
+    }
+    __syncthreads();
+    if (tt >= tps) return;
+    uint32_t m[8], lo_at[8], lo_w[8];
+    int off[8], at[8];
+    float f[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int rl = s_role[8 * j + e];
+        const bool src = rl >= 0, don = rl <= -2;
+        f[e] = don ? s_pad[-rl - 2] : s_scale[8 * j + e];
+        m[e] = src ? 16u : don ? 0u : 1u;
+        off[e] = src ? 128 : don ? -1 : 8;
+        lo_w[e] = src ? 4u : 0u;
+        lo_at[e] = src ? 4u * (uint32_t)(rl & 7) : 0u;
+        at[e] = tt * L + (src ? rl >> 3 : j);
+    }
+    const int64_t obase = out_row(a, row) + 8 * j;
+#pragma unroll
+    for (int i = 0; i < KW_STEPS; ++i) {
+        const int64_t t = t0 + i * tps;
+        if (t >= a.T) return;
+        const uint32_t w = s_word[i][tid];
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t lo = __builtin_amdgcn_ubfe(s_word[i][at[e]], lo_at[e], lo_w[e]);
+            const int code = (int)(__umul24(__builtin_amdgcn_ubfe(w, 4 * e, 4), m[e]) + lo) - off[e];
+            v[e] = __fmul_rn((float)code, f[e]);
+        }
+        if constexpr (OUT == IQ_F32) {
+            float4 *o = (float4 *)((float *)a.out + obase + t * D);
+            o[0] = float4{v[0], v[1], v[2], v[3]};
+            o[1] = float4{v[4], v[5], v[6], v[7]};
+        } else {
+            uint32_t h[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) h[k] = pack_pair<OUT>(v[2 * k], v[2 * k + 1]);
+            __builtin_nontemporal_store(u32x4_nt{h[0], h[1], h[2], h[3]}, (u32x4_nt *)((uint16_t *)a.out + obase + t * D));
         }
     }
 }
@@ -477,36 +571,115 @@ extern "C" int iq_v_quantize(const void *x, int x_dtype, const int64_t *x_stride
     return IQ_OK;
 }
 
-extern "C" int iq_v_dequantize(const uint8_t *payload, const uint16_t *scales, const uint16_t *offsets,
-                               int64_t rows, int64_t D, int bits, int group, void *out, int out_dtype, void *stream)
+namespace {
+
+// element strides and base of a dense output whose rows take 16-byte stores
+bool out_vec(const void *out, int out_dtype, int64_t D, int64_t osb, int64_t osh)
+{
+    const int64_t v = out_dtype == IQ_F32 ? 4 : 8;
+    return ((uintptr_t)out & 15) == 0 && D % v == 0 && osb % v == 0 && osh % v == 0;
+}
+
+template <int BITS, int OUT>
+void launch_v_rows(const VDecArgs &a, int64_t rows, hipStream_t st)
+{
+    const dim3 grid((unsigned)((a.T * (a.D / 16) + V_THREADS - 1) / V_THREADS), (unsigned)rows), block(V_THREADS);
+    if (a.D == 128) hipLaunchKernelGGL((v_decode_rows<BITS, OUT, 8>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((v_decode_rows<BITS, OUT, 0>), grid, block, 0, st, a);
+}
+
+template <int BITS>
+void launch_v_rows(const VDecArgs &a, int64_t rows, hipStream_t st)
+{
+    if (a.out_dt == IQ_BF16) launch_v_rows<BITS, IQ_BF16>(a, rows, st);
+    else if (a.out_dt == IQ_F16) launch_v_rows<BITS, IQ_F16>(a, rows, st);
+    else launch_v_rows<BITS, IQ_F32>(a, rows, st);
+}
+
+}  // namespace
+
+extern "C" int iq_v_dequantize_into(const uint8_t *payload, const uint16_t *scales, const uint16_t *offsets, int64_t B,
+                                    int64_t H, int64_t T, int64_t D, int bits, int group, void *out, int out_dtype,
+                                    int64_t out_sb, int64_t out_sh, void *stream)
 {
     IQ_CHECK_ARG(bits == 2 || bits == 4, "iq_v_dequantize: bits must be 2 or 4");
     IQ_CHECK_ARG(group == 32 || group == 64 || group == 128, "iq_v_dequantize: bad group");
-    IQ_CHECK_ARG(rows >= 0 && D >= group && D % group == 0, "iq_v_dequantize: bad shape");
+    IQ_CHECK_ARG(B >= 0 && H >= 1 && T >= 0 && D >= group && D % group == 0, "iq_v_dequantize: bad shape");
     IQ_CHECK_ARG(out_dtype >= IQ_F32 && out_dtype <= IQ_F16, "iq_v_dequantize: bad out dtype");
-    if (rows == 0) return IQ_OK;
+    if (B == 0 || T == 0) return IQ_OK;
     IQ_CHECK_ARG(payload && scales && offsets && out, "iq_v_dequantize: null pointer");
-    const int64_t n = rows * D;
-    VDecArgs a{payload, scales, offsets, rows, D, bits, group, out, out_dtype};
-    if (D == 128 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)payload & (bits == 2 ? 3 : 7)) == 0 &&
-        (rows * 8 + V_THREADS - 1) / V_THREADS <= 0x7fffffffLL) {
-        const dim3 grid((unsigned)((rows * 8 + V_THREADS - 1) / V_THREADS)), block(V_THREADS);
-        const hipStream_t st = (hipStream_t)stream;
-        if (bits == 2) {
-            if (out_dtype == IQ_BF16) hipLaunchKernelGGL((v_decode_rows<2, IQ_BF16>), grid, block, 0, st, a);
-            else if (out_dtype == IQ_F16) hipLaunchKernelGGL((v_decode_rows<2, IQ_F16>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((v_decode_rows<2, IQ_F32>), grid, block, 0, st, a);
-        } else {
-            if (out_dtype == IQ_BF16) hipLaunchKernelGGL((v_decode_rows<4, IQ_BF16>), grid, block, 0, st, a);
-            else if (out_dtype == IQ_F16) hipLaunchKernelGGL((v_decode_rows<4, IQ_F16>), grid, block, 0, st, a);
-            else hipLaunchKernelGGL((v_decode_rows<4, IQ_F32>), grid, block, 0, st, a);
-        }
+    IQ_CHECK_ARG(H <= 65535 && T * D <= 0x7fffffffLL * V_THREADS, "iq_v_dequantize: too large");
+    const int64_t most = 65535 / H;             // a launch's batches (rows are the grid's y)
+    for (; B > most; B -= most) {
+        const int rc = iq_v_dequantize_into(payload, scales, offsets, most, H, T, D, bits, group, out, out_dtype, out_sb,
+                                            out_sh, stream);
+        if (rc != IQ_OK) return rc;
+        const int64_t tokens = most * H * T;
+        payload += tokens * (D * bits / 8);
+        scales += tokens * (D / group);
+        offsets += tokens * (D / group);
+        out = (char *)out + most * out_sb * (out_dtype == IQ_F32 ? 4 : 2);
+    }
+    const VDecArgs a{payload, scales, offsets, H, T, D, bits, group, out, out_dtype, out_sb, out_sh};
+    const hipStream_t st = (hipStream_t)stream;
+    if (out_vec(out, out_dtype, D, out_sb, out_sh) && ((uintptr_t)payload & (bits == 2 ? 3 : 7)) == 0 &&
+        T * (D / 16) <= 0x7fffffffLL) {
+        if (bits == 2) launch_v_rows<2>(a, B * H, st);
+        else launch_v_rows<4>(a, B * H, st);
         IQ_CHECK_LAUNCH("v_decode_rows");
         return IQ_OK;
     }
-    hipLaunchKernelGGL(v_decode_kernel, dim3((unsigned)((n + V_THREADS - 1) / V_THREADS)), dim3(V_THREADS), 0,
-                       (hipStream_t)stream, a);
+    hipLaunchKernelGGL(v_decode_kernel, dim3((unsigned)((T * D + V_THREADS - 1) / V_THREADS), (unsigned)(B * H)),
+                       dim3(V_THREADS), 0, st, a);
     IQ_CHECK_LAUNCH("v_decode_kernel");
+    return IQ_OK;
+}
+
+extern "C" int iq_v_dequantize(const uint8_t *payload, const uint16_t *scales, const uint16_t *offsets,
+                               int64_t rows, int64_t D, int bits, int group, void *out, int out_dtype, void *stream)
+{
+    // one row of `rows` tokens
+    return iq_v_dequantize_into(payload, scales, offsets, 1, 1, rows, D, bits, group, out, out_dtype, 0, 0, stream);
+}
+
+extern "C" int iq_k4_dequantize_into(const uint8_t *payload, const float *scales, const void *src, const void *don,
+                                     int desc_bytes, const float *padding, int64_t B, int64_t H, int64_t T, int64_t D,
+                                     int64_t count, void *out, int out_dtype, int64_t out_sb, int64_t out_sh,
+                                     void *stream)
+{
+    IQ_CHECK_ARG(D >= 2 && D % 2 == 0 && D <= 1024, "iq_k4_dequantize: bad D");
+    IQ_CHECK_ARG(count >= 0 && 2 * count <= D, "iq_k4_dequantize: bad count");
+    IQ_CHECK_ARG(desc_bytes == 1 || desc_bytes == 4 || desc_bytes == 8, "iq_k4_dequantize: desc_bytes");
+    IQ_CHECK_ARG(out_dtype >= IQ_F32 && out_dtype <= IQ_F16, "iq_k4_dequantize: bad out dtype");
+    IQ_CHECK_ARG(B >= 0 && H >= 1 && T >= 0, "iq_k4_dequantize: bad shape");
+    const int64_t rows = B * H;
+    if (rows == 0 || T == 0) return IQ_OK;
+    IQ_CHECK_ARG(payload && scales && out && (count == 0 || (src && don && padding)), "iq_k4_dequantize: null");
+    IQ_CHECK_ARG(rows * T <= 0x7fffffffLL, "iq_k4_dequantize: too large");
+    const KDecArgs a{payload, scales, src, don, desc_bytes, padding, rows, T, D, count, out, out_dtype, H, out_sb, out_sh};
+    const dim3 block(V_THREADS);
+    const hipStream_t st = (hipStream_t)stream;
+    const bool vec = out_vec(out, out_dtype, D, out_sb, out_sh) && ((uintptr_t)payload & 3) == 0 && rows <= 65535 &&
+                     D % 8 == 0;
+    if (vec && D == 128 && desc_bytes == 1 && count <= 64) {
+        const dim3 grid((unsigned)((T + KD_TOKENS - 1) / KD_TOKENS), (unsigned)rows);
+        if (out_dtype == IQ_BF16) hipLaunchKernelGGL((k4_decode_rows<IQ_BF16>), grid, block, 0, st, a);
+        else if (out_dtype == IQ_F16) hipLaunchKernelGGL((k4_decode_rows<IQ_F16>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k4_decode_rows<IQ_F32>), grid, block, 0, st, a);
+        IQ_CHECK_LAUNCH("k4_decode_rows");
+        return IQ_OK;
+    }
+    if (vec) {
+        const int64_t tile = KW_STEPS * (V_THREADS / (D / 8));
+        const dim3 grid((unsigned)((T + tile - 1) / tile), (unsigned)rows);
+        if (out_dtype == IQ_BF16) hipLaunchKernelGGL((k4_decode_words<IQ_BF16>), grid, block, 0, st, a);
+        else if (out_dtype == IQ_F16) hipLaunchKernelGGL((k4_decode_words<IQ_F16>), grid, block, 0, st, a);
+        else hipLaunchKernelGGL((k4_decode_words<IQ_F32>), grid, block, 0, st, a);
+        IQ_CHECK_LAUNCH("k4_decode_words");
+        return IQ_OK;
+    }
+    hipLaunchKernelGGL(k4_decode_kernel, dim3((unsigned)(rows * T)), block, 0, st, a);
+    IQ_CHECK_LAUNCH("k4_decode_kernel");
     return IQ_OK;
 }
 
@@ -514,26 +687,6 @@ extern "C" int iq_k4_dequantize(const uint8_t *payload, const float *scales, con
                                 int desc_bytes, const float *padding, int64_t rows, int64_t T, int64_t D,
                                 int64_t count, void *out, int out_dtype, void *stream)
 {
-    IQ_CHECK_ARG(D >= 2 && D % 2 == 0 && D <= 1024, "iq_k4_dequantize: bad D");
-    IQ_CHECK_ARG(count >= 0 && 2 * count <= D, "iq_k4_dequantize: bad count");
-    IQ_CHECK_ARG(desc_bytes == 1 || desc_bytes == 4 || desc_bytes == 8, "iq_k4_dequantize: desc_bytes");
-    IQ_CHECK_ARG(out_dtype >= IQ_F32 && out_dtype <= IQ_F16, "iq_k4_dequantize: bad out dtype");
-    IQ_CHECK_ARG(rows >= 0 && T >= 0, "iq_k4_dequantize: bad shape");
-    if (rows == 0 || T == 0) return IQ_OK;
-    IQ_CHECK_ARG(payload && scales && out && (count == 0 || (src && don && padding)), "iq_k4_dequantize: null");
-    IQ_CHECK_ARG(rows * T <= 0x7fffffffLL, "iq_k4_dequantize: too large");
-    KDecArgs a{payload, scales, src, don, desc_bytes, padding, rows, T, D, count, out, out_dtype};
-    if (D == 128 && desc_bytes == 1 && count <= 64 && ((uintptr_t)out & 15) == 0 && ((uintptr_t)payload & 3) == 0 &&
-        rows <= 65535 && out_dtype != IQ_F64) {
-        const dim3 grid((unsigned)((T + KD_TOKENS - 1) / KD_TOKENS), (unsigned)rows), block(V_THREADS);
-        const hipStream_t st = (hipStream_t)stream;
-        if (out_dtype == IQ_BF16) hipLaunchKernelGGL((k4_decode_rows<IQ_BF16>), grid, block, 0, st, a);
-        else if (out_dtype == IQ_F16) hipLaunchKernelGGL((k4_decode_rows<IQ_F16>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((k4_decode_rows<IQ_F32>), grid, block, 0, st, a);
-        IQ_CHECK_LAUNCH("k4_decode_rows");
-        return IQ_OK;
-    }
-    hipLaunchKernelGGL(k4_decode_kernel, dim3((unsigned)(rows * T)), dim3(V_THREADS), 0, (hipStream_t)stream, a);
-    IQ_CHECK_LAUNCH("k4_decode_kernel");
-    return IQ_OK;
+    return iq_k4_dequantize_into(payload, scales, src, don, desc_bytes, padding, rows, 1, T, D, count, out, out_dtype,
+                                 T * D, 0, stream);
 }

@@ -45,6 +45,12 @@ class TailDesc(ctypes.Structure):
                 ("flag", ctypes.c_uint64), ("k_sh", _i64), ("k_st", _i64), ("v_sh", _i64), ("v_st", _i64)]
 
 
+class CopySegment(ctypes.Structure):
+    """Mirror of iq_copy_segment in include/inquant_hip.h."""
+    _fields_ = [("src", ctypes.c_uint64), ("dst", ctypes.c_uint64), ("src_h", _i64), ("src_t", _i64),
+                ("dst_h", _i64), ("dst_t", _i64), ("tokens", _i64)]
+
+
 _SIGNATURES = {
     "iq_abi_version": (_int, []),
     "iq_last_error": (ctypes.c_char_p, []),
@@ -52,6 +58,10 @@ _SIGNATURES = {
                               _p, _p, _p, _p, _int, _p, _p, _p]),
     "iq_reuse_map": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _p]),
     "iq_k4_dequantize": (_int, [_p, _p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _p, _int, _p]),
+    "iq_k4_dequantize_into": (_int, [_p, _p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _i64, _i64,
+                                     _p]),
+    "iq_v_dequantize_into": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _int, _int, _p, _int, _i64, _i64, _p]),
+    "iq_copy_rows": (_int, [ctypes.POINTER(CopySegment), _i64, _i64, _i64, _p]),
     "iq_v_quantize": (_int, [_p, _int, ctypes.POINTER(_i64), _i64, _i64, _i64, _i64, _int, _int,
                              _p, _p, _p, _p, _p]),
     "iq_v_dequantize": (_int, [_p, _p, _p, _i64, _i64, _int, _int, _p, _int, _p]),

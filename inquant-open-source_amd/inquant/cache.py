@@ -108,6 +108,25 @@ class PackedAttentionView(NamedTuple):
     seq_length: int
 
 
+def _copy_rows(pairs) -> None:
+    """Copies (source, destination) pairs of [1, H, n, D] views, at most eight
+    and of one head count, width and dtype, in one launch."""
+    first = pairs[0][0]
+    if not first.is_cuda or any(s.stride(3) != 1 or d.stride(3) != 1 for s, d in pairs):
+        for s, d in pairs:
+            d.copy_(s)
+        return
+    eb = first.element_size()
+    segments = (nat.CopySegment * len(pairs))()
+    for g, (s, d) in zip(segments, pairs):
+        _, sh, st, _ = s.stride()
+        _, dh, dt, _ = d.stride()
+        g.src, g.dst, g.src_h, g.src_t = s.data_ptr(), d.data_ptr(), sh * eb, st * eb
+        g.dst_h, g.dst_t, g.tokens = dh * eb, dt * eb, s.shape[2]
+    nat.check(nat.lib().iq_copy_rows(segments, len(pairs), first.shape[1], first.shape[3] * eb,
+                                     nat.stream_handle(first.device)))
+
+
 class _Rows:
     """A [2, H, capacity, D] buffer of dense rows; keys at [0], values at [1]."""
 
@@ -149,8 +168,7 @@ class _Rows:
         if self.start + self.count + n > self.capacity:
             self.compact()
         end = self.start + self.count
-        self.buf[0:1, :, end:end + n].copy_(keys)
-        self.buf[1:2, :, end:end + n].copy_(values)
+        _copy_rows([(keys, self.kbuf[:, :, end:end + n]), (values, self.vbuf[:, :, end:end + n])])
 
     def compact(self) -> None:
         if self.start:
@@ -272,6 +290,28 @@ def _run_block(blocks, i: int, j: int):
         return PackedValues(**fields, shape=shape, original_dtype=first.original_dtype, bits=first.bits,
                             group_size=first.group_size)
     return PackedTensor(**fields, shape=shape, original_dtype=first.original_dtype)
+
+
+def _dequantize_into(run, dense, at: int) -> None:
+    """The blocks of a run [n, H, T, D] dequantized to token rows at .. at + n T
+    of a contiguous dense [1, H, tokens, D]."""
+    n, heads, T, dim = run.shape
+    if dense.dtype not in _SEAL_DTYPES:
+        rows = dense[:, :, at:at + n * T].unflatten(2, (n, T))
+        rows.copy_(run.dequantize(dtype=dense.dtype).permute(1, 0, 2, 3).unsqueeze(0))
+        return
+    place = (dense.data_ptr() + at * dim * dense.element_size(), nat.dtype_code(dense.dtype), T * dim, dense.stride(1),
+             nat.stream_handle(dense.device))
+    if isinstance(run, PackedValues):
+        nat.check(nat.lib().iq_v_dequantize_into(
+            run.payload.data_ptr(), run.scales.data_ptr(), run.offsets.data_ptr(), n, heads, T, dim, run.bits,
+            run.group_size, *place))
+        return
+    count = run.salient_channels.shape[-1]
+    src, don, padding = (t.data_ptr() if count else None for t in (run.salient_channels, run.donor_channels, run.padding))
+    nat.check(nat.lib().iq_k4_dequantize_into(
+        run.payload.data_ptr(), run.scales.data_ptr(), src, don, run.salient_channels.element_size(), padding, n, heads,
+        T, dim, count, *place))
 
 
 _SEAL_DTYPES = (torch.float32, torch.bfloat16, torch.float16)   # what the batched seal encoders read
@@ -738,25 +778,25 @@ class InQuantCache(_HFCache):
         sink_n = 0 if layer.sink is None else layer.sink.count
         tail_n = 0 if layer.tail is None else layer.tail.count
         new_n = 0 if new_keys is None else new_keys.shape[2]
-        out = []
+        packed = sum(b.shape[2] for b in layer.key_blocks)
+        total = sink_n + packed + tail_n + new_n
+        out, pairs = [], []
         for side, blocks in ((0, layer.key_blocks), (1, layer.value_blocks)):
-            total = sink_n + sum(b.shape[2] for b in blocks) + tail_n + new_n
             dense = torch.empty((1, heads, total, dim), dtype=layer.dtype, device=layer.device)
-            at = 0
             if sink_n:
-                rows = layer.sink
-                dense[:, :, :sink_n].copy_(rows.buf[side:side + 1, :, rows.start:rows.start + sink_n])
-                at = sink_n
+                pairs.append((layer.sink.values() if side else layer.sink.keys(), dense[:, :, :sink_n]))
+            at = sink_n
             for i, j in layer.runs:
-                n, T = j - i, blocks[i].shape[2]
-                deq = _run_block(blocks, i, j).dequantize(dtype=layer.dtype)     # [n, H, T, D]
-                dense[:, :, at:at + n * T].view(1, heads, n, T, dim).copy_(deq.permute(1, 0, 2, 3).unsqueeze(0))
-                at += n * T
+                run = _run_block(blocks, i, j)                           # [n, H, T, D]
+                _dequantize_into(run, dense, at)
+                at += (j - i) * run.shape[2]
             if tail_n:
-                dense[:, :, at:at + tail_n].copy_(layer.tail.keys() if side == 0 else layer.tail.values())
+                pairs.append((layer.tail.values() if side else layer.tail.keys(), dense[:, :, at:at + tail_n]))
             if new_n:
-                dense[:, :, at + tail_n:].copy_(new_keys if side == 0 else new_values)
+                pairs.append((new_values if side else new_keys, dense[:, :, at + tail_n:]))
             out.append(dense)
+        if pairs:
+            _copy_rows(pairs)
         return out[0], out[1]
 
     # ------------------------------------------------------------ accounting (cache.py:346-394)

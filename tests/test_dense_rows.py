@@ -1,0 +1,49 @@
+"""Packed blocks dequantized into their place of a dense history, at head sizes
+and lengths around the tiles of the row kernels, and copies of dense rows."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle
+import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D,T", [(8, 37), (32, 1), (64, 129), (96, 85), (128, 130), (256, 33), (1024, 9), (66, 20)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_k4_dequantize_sizes(D, T, dtype):
+    from inquant.codec import CodecConfig, quantize
+    x = torch.from_numpy(synth.normal(D + T, (2, 3, T, D))).cuda().to(dtype)
+    packed = quantize(x, CodecConfig(salient_fraction=0.25))
+    want = oracle.k4_dequantize({k: v.cpu().numpy() for k, v in packed.tensors.items()}, str(dtype)[6:])
+    assert torch.equal(packed.dequantize().float().cpu(), torch.from_numpy(want))
+
+
+@pytest.mark.parametrize("D,block,vbits,group,dtype", [
+    (128, 256, 2, 64, torch.bfloat16), (64, 64, None, 64, torch.float16), (64, 48, 4, 32, torch.float32),
+    (96, 100, 2, 32, torch.bfloat16), (66, 32, None, 32, torch.float16), (256, 32, 4, 128, torch.bfloat16)])
+def test_materialize_places_every_block(D, block, vbits, group, dtype):
+    from inquant.cache import CacheConfig, InQuantCache
+    cache = InQuantCache(CacheConfig(block_size=block, residual_length=16, sink_tokens=3, value_bits=vbits,
+                                     value_group_size=group))
+    x = torch.from_numpy(synth.normal(D + block, (2, 5 * block + 40, 2, D))).cuda().to(dtype)
+    k, v = x[0].transpose(0, 1)[None], x[1].transpose(0, 1)[None]
+    cache.update(k[:, :, :3 * block + 30], v[:, :, :3 * block + 30], 0)
+    cache.update(k[:, :, 3 * block + 30:], v[:, :, 3 * block + 30:], 0)       # a second run of blocks
+    layer = cache._layers[0]
+    for got, blocks, whole in zip(cache.materialize(0), (layer.key_blocks, layer.value_blocks), (k, v)):
+        packed = [b.dequantize(dtype=dtype) for b in blocks]
+        at = 3 + block * len(blocks)
+        assert torch.equal(got, torch.cat([whole[:, :, :3], *packed, whole[:, :, at:]], 2))
+
+
+@pytest.mark.parametrize("offset,width", [(0, 64), (1, 64), (2, 62), (0, 3)])
+def test_copied_rows(offset, width):
+    from inquant.cache import _copy_rows
+    src = torch.randn(1, 3, 37, 80, device="cuda").bfloat16()
+    dst = torch.zeros(1, 3, 50, 80, device="cuda").bfloat16()
+    a, b = src[:, :, :20, offset:offset + width], src[:, :, 20:, offset:offset + width]
+    _copy_rows([(a, dst[:, :, 25:45, :width]), (b, dst[:, :, :17, :width]), (a[:, :, :0], dst[:, :, :0, :width])])
+    assert torch.equal(dst[:, :, 25:45, :width], a) and torch.equal(dst[:, :, :17, :width], b)
+    assert np.count_nonzero(dst.float().cpu().numpy()) <= 3 * 37 * width
