@@ -24,6 +24,7 @@
  *   iq_k4_dequantize    src/inquant/codec.py:112-134         PackedTensor.dequantize()
  *   iq_k4_dequantize_into, iq_v_dequantize_into, iq_copy_rows
  *                       src/inquant/cache.py:328-345         InQuantCache materialize
+ *   iq_check_positions  src/inquant/cache.py:230-240         the contiguous-append position check
  *   iq_v_quantize       src/inquant/value_codec.py:51-72     quantize_values()
  *   iq_v_dequantize     src/inquant/value_codec.py:38-48     PackedValues.dequantize()
  *   iq_kv_quantize      src/inquant/cache.py:288-295 (the paired key / value block
@@ -424,6 +425,13 @@ typedef struct iq_tail_desc {
 
 int iq_tail_append_row(const iq_tail_desc *desc, const void *k, const void *v, int64_t slot, int64_t shift_src,
                        int64_t shift_count, const void *positions, int64_t expected, void *stream);
+
+/*
+ * Sets *flag unless position i (int32 or int64, every stride-th) is
+ * expected + i for all i < n (cache.py:230-240).
+ */
+int iq_check_positions(const void *positions, int pos_bytes, int64_t stride, int64_t n, int64_t expected, int *flag,
+                       void *stream);
 
 /*
  * Copies of [H, tokens] rows of row_bytes bytes, up to IQ_COPY_SEGMENTS

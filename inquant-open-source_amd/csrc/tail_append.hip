@@ -79,6 +79,15 @@ __global__ __launch_bounds__(256) void copy_rows_kernel(CopyArgs a)
     for (int64_t u = threadIdx.x & 15; u < a.row_units; u += 16) dst[u] = src[u];
 }
 
+__global__ __launch_bounds__(256) void check_positions_kernel(const void *pos, int bytes, int64_t stride, int64_t n,
+                                                              int64_t expected, int *flag)
+{
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n) return;
+    const int64_t got = bytes == 8 ? ((const int64_t *)pos)[i * stride] : (int64_t)((const int32_t *)pos)[i * stride];
+    if (got != expected + i) *flag = 1;
+}
+
 }  // namespace
 
 extern "C" int iq_tail_append(const void *k, const void *v, int64_t k_sh, int64_t k_st, int64_t v_sh, int64_t v_st,
@@ -184,5 +193,18 @@ extern "C" int iq_copy_rows(const iq_copy_segment *segments, int64_t n, int64_t 
         hipLaunchKernelGGL(copy_rows_kernel<uint8_t>, grid, block, 0, s, a);
     }
     IQ_CHECK_LAUNCH("copy_rows_kernel");
+    return IQ_OK;
+}
+
+extern "C" int iq_check_positions(const void *positions, int pos_bytes, int64_t stride, int64_t n, int64_t expected,
+                                  int *flag, void *stream)
+{
+    IQ_CHECK_ARG(n >= 0 && (n == 0 || positions) && flag && (pos_bytes == 4 || pos_bytes == 8),
+                 "iq_check_positions: bad arguments");
+    IQ_CHECK_ARG((n + 255) / 256 <= 0x7fffffffLL, "iq_check_positions: too many positions");
+    if (n == 0) return IQ_OK;
+    hipLaunchKernelGGL(check_positions_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                       positions, pos_bytes, stride, n, expected, flag);
+    IQ_CHECK_LAUNCH("check_positions_kernel");
     return IQ_OK;
 }

@@ -61,6 +61,7 @@ _SIGNATURES = {
     "iq_k4_dequantize_into": (_int, [_p, _p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _i64, _i64,
                                      _p]),
     "iq_v_dequantize_into": (_int, [_p, _p, _p, _i64, _i64, _i64, _i64, _int, _int, _p, _int, _i64, _i64, _p]),
+    "iq_check_positions": (_int, [_p, _int, _i64, _i64, _i64, _p, _p]),
     "iq_copy_rows": (_int, [ctypes.POINTER(CopySegment), _i64, _i64, _i64, _p]),
     "iq_v_quantize": (_int, [_p, _int, ctypes.POINTER(_i64), _i64, _i64, _i64, _i64, _int, _int,
                              _p, _p, _p, _p, _p]),

@@ -52,7 +52,7 @@ except ImportError:  # the codec and cache do not need transformers
 
 from . import _native as nat
 from .codec import _BAD_K, CodecConfig, PackedTensor, _per_block, quantize
-from .value_codec import _BAD_V, PackedValues, _value_blocks
+from .value_codec import _BAD_V, PackedValues, quantize_values
 
 _POSITION_ERROR = "Only contiguous append positions are supported; reset before a new request"
 
@@ -187,13 +187,39 @@ class _LayerCache:
         self.seq_length = 0
         self.sink: _Rows | None = None
         self.tail: _Rows | None = None
-        self.key_blocks: list = []
-        self.value_blocks: list = []
         self.runs: list = []            # [first, stop) of the blocks of each seal (one batched encode)
+        self.batches: list = []         # its (keys, values), batched [stop - first, H, T, D]
+        self._keys: list = []           # the blocks of the first batches, as objects
+        self._values: list = []
         self.packed_nbytes = 0
         self.full_sink = None          # (keys, values) views once the sink holds all its rows
         self.block_tuples = None       # (key blocks, value blocks) as tuples, rebuilt after a seal
         self.seal_out = None           # outputs of the next one-block seal, carved ahead of it
+
+    @property
+    def block_count(self) -> int:
+        return self.runs[-1][1] if self.runs else 0
+
+    def _expand(self) -> None:
+        """Block objects of the batches that have none yet: a prefill's blocks
+        are 16 views and two objects each (0.6 ms for 127 of them), which only
+        a reader of single blocks needs."""
+        for (first, stop), (keys, values) in zip(self.runs, self.batches):
+            if first == len(self._keys):
+                self._keys.extend(_unbatched(keys, stop - first))
+                self._values.extend(_unbatched(values, stop - first))
+
+    @property
+    def key_blocks(self) -> list:
+        if len(self._keys) != self.block_count:
+            self._expand()
+        return self._keys
+
+    @property
+    def value_blocks(self) -> list:
+        if len(self._keys) != self.block_count:
+            self._expand()
+        return self._values
 
     # the reference's field names, as views of the rows
     @property
@@ -227,6 +253,11 @@ class _LayerCache:
         return 0 if self.seal_out is None else self.seal_out[0].untyped_storage().nbytes()
 
 
+def _blocked(tensor: torch.Tensor, block_count: int, block_size: int) -> torch.Tensor:
+    """The [blocks, H, B, D] view of the first blocks of [1, H, T, D]."""
+    return tensor[0, :, :block_count * block_size].unflatten(1, (block_count, block_size)).transpose(0, 1)
+
+
 def _quantize_temporal_blocks(tensor: torch.Tensor, block_count: int, block_size: int,
                               config: CodecConfig, bad: torch.Tensor | None = None) -> list[PackedTensor]:
     """K4-encode the first ``block_count`` blocks of [1, H, T, D] as
@@ -236,8 +267,7 @@ def _quantize_temporal_blocks(tensor: torch.Tensor, block_count: int, block_size
     if block_count == 0:
         return []
     _, heads, _, dim = tensor.shape
-    blocked = tensor[0, :, :block_count * block_size].unflatten(1, (block_count, block_size)).transpose(0, 1)
-    packed = quantize(blocked, config, _flag=bad)
+    packed = quantize(_blocked(tensor, block_count, block_size), config, _flag=bad)
     return _per_block(packed, block_count, (1, heads, block_size, dim), PackedTensor)
 
 
@@ -275,21 +305,14 @@ def _carve(device, fields):
     return [torch.as_strided(typed[i], shape, strides, offset) for i, shape, strides, offset in views]
 
 
-def _run_block(blocks, i: int, j: int):
-    """blocks[i:j], the per-block views of one batched encode (consecutive
-    equal-size slices of each field's allocation), as one batched
-    [j - i, H, T, D] block over the same memory."""
-    first = blocks[i]
-    if j - i == 1:
-        return first
-    n = j - i
-    fields = {name: torch.as_strided(t, (n, *t.shape[1:]), (t.numel(), *t.stride()[1:]), t.storage_offset())
-              for name, t in first.tensors.items()}
-    shape = (n, *first.shape[1:])
-    if isinstance(first, PackedValues):
-        return PackedValues(**fields, shape=shape, original_dtype=first.original_dtype, bits=first.bits,
-                            group_size=first.group_size)
-    return PackedTensor(**fields, shape=shape, original_dtype=first.original_dtype)
+def _unbatched(batch, count: int) -> list:
+    """The blocks of a batched [count, H, T, D] encode, views of its fields."""
+    if count == 1:
+        return [batch]
+    shape = (1, *batch.shape[1:])
+    if isinstance(batch, PackedValues):
+        return _per_block(batch, count, shape, PackedValues, bits=batch.bits, group_size=batch.group_size)
+    return _per_block(batch, count, shape, PackedTensor)
 
 
 def _dequantize_into(run, dense, at: int) -> None:
@@ -356,17 +379,15 @@ def _kv_blocks(keys: torch.Tensor, values: torch.Tensor, block_count: int, block
     """K4 keys and group-wise values of the first ``block_count`` blocks of
     [1, H, T, D] in one library call (iq_kv_quantize: one launch for sealed
     256-token blocks of 128 16-bit channels, the two encoders back to back
-    otherwise), with the per-block objects and flags of
-    _quantize_temporal_blocks + _value_blocks (cache.py:288-295).  ``out``:
-    the outputs as carved for _seal_fields, allocated beforehand."""
-    if block_count == 0:
-        return [], []
+    otherwise), batched [blocks, H, B, D], with the flags of
+    quantize + quantize_values (cache.py:288-295).  ``out``: the outputs as
+    carved for _seal_fields, allocated beforehand."""
     _, heads, _, dim = keys.shape
     native = (keys.dtype == values.dtype and keys.dtype in _SEAL_DTYPES and keys.shape == values.shape
               and _seal_native(dim, bits, group_size))
     if not native:      # the separate encoders, with their own argument errors
-        return (_quantize_temporal_blocks(keys, block_count, block_size, config, key_flag),
-                _value_blocks(values, block_count, block_size, bits, group_size, value_flag))
+        return (quantize(_blocked(keys, block_count, block_size), config, _flag=key_flag),
+                quantize_values(_blocked(values, block_count, block_size), bits, group_size, _flag=value_flag))
     device = nat.require_gpu(keys, what="quantize")
     # the [blocks, H, B, D] view of the first blocks, as pointer and strides
     # (no view objects: the encoder reads them directly)
@@ -383,31 +404,23 @@ def _kv_blocks(keys: torch.Tensor, values: torch.Tensor, block_count: int, block
         src.element_size(), padding.data_ptr() if count else None, bits, group_size, v_payload.data_ptr(),
         v_scales.data_ptr(), v_offsets.data_ptr(), key_flag.data_ptr(), value_flag.data_ptr(),
         nat.stream_handle(device)))
-    shape = (1, heads, block_size, dim)
-    if B == 1:          # a seal's one block: the objects directly
-        return ([PackedTensor(payload, scales, src, don, padding, shape, keys.dtype)],
-                [PackedValues(v_payload, v_scales, v_offsets, shape, values.dtype, bits, group_size)])
-    packed_k = PackedTensor(payload, scales, src, don, padding, (B, H, T, D), keys.dtype)
-    packed_v = PackedValues(v_payload, v_scales, v_offsets, (B, H, T, D), values.dtype, bits, group_size)
-    return (_per_block(packed_k, block_count, shape, PackedTensor),
-            _per_block(packed_v, block_count, shape, PackedValues, bits=bits, group_size=group_size))
+    return (PackedTensor(payload, scales, src, don, padding, (B, H, T, D), keys.dtype),
+            PackedValues(v_payload, v_scales, v_offsets, (B, H, T, D), values.dtype, bits, group_size))
 
 
 def _k4_pair_blocks(keys: torch.Tensor, values: torch.Tensor, block_count: int, block_size: int,
                     config: CodecConfig, key_flag: torch.Tensor, value_flag: torch.Tensor, out=None):
     """K4 keys and K4-coded values (value_bits None) of the first
     ``block_count`` blocks in one library call (iq_k4_quantize_kv: one launch
-    for 16-bit blocks of 128 channels), with the per-block objects and flags
-    of two _quantize_temporal_blocks calls (cache.py:288-291).  ``out`` as
-    for _kv_blocks."""
-    if block_count == 0:
-        return [], []
+    for 16-bit blocks of 128 channels), batched [blocks, H, B, D], with the
+    flags of two quantize calls (cache.py:288-291).  ``out`` as for
+    _kv_blocks."""
     _, heads, _, dim = keys.shape
     native = (keys.dtype == values.dtype and keys.dtype in _SEAL_DTYPES and keys.shape == values.shape
               and _seal_native(dim, None, 0))
     if not native:      # the separate encodes, with their own argument errors
-        return (_quantize_temporal_blocks(keys, block_count, block_size, config, key_flag),
-                _quantize_temporal_blocks(values, block_count, block_size, config, value_flag))
+        return (quantize(_blocked(keys, block_count, block_size), config, _flag=key_flag),
+                quantize(_blocked(values, block_count, block_size), config, _flag=value_flag))
     device = nat.require_gpu(keys, what="quantize")
     B, H, T, D = block_count, heads, block_size, dim
     k_strides = _block_strides(keys.stride(), T)
@@ -420,11 +433,7 @@ def _k4_pair_blocks(keys: torch.Tensor, values: torch.Tensor, block_count: int, 
         keys.data_ptr(), values.data_ptr(), nat.dtype_code(keys.dtype), k_strides, v_strides, B, H, T, D,
         count, config.sample_stride, int(config.donor_policy == "min_error"), *ptrs(ko), *ptrs(vo),
         ko[2].element_size(), key_flag.data_ptr(), value_flag.data_ptr(), nat.stream_handle(device)))
-    shape = (1, heads, block_size, dim)
-    if B == 1:          # a seal's one block: the objects directly
-        return [PackedTensor(*ko, shape, keys.dtype)], [PackedTensor(*vo, shape, values.dtype)]
-    return (_per_block(PackedTensor(*ko, (B, H, T, D), keys.dtype), block_count, shape, PackedTensor),
-            _per_block(PackedTensor(*vo, (B, H, T, D), values.dtype), block_count, shape, PackedTensor))
+    return PackedTensor(*ko, (B, H, T, D), keys.dtype), PackedTensor(*vo, (B, H, T, D), values.dtype)
 
 
 class InQuantCache(_HFCache):
@@ -516,15 +525,28 @@ class InQuantCache(_HFCache):
             self._flags = torch.zeros(3, dtype=torch.int32, device=device)
         return self._flags
 
-    def _host_position_check(self, position: torch.Tensor, start: int) -> None:
-        """Synchronous comparison with start, start + 1, ... (raises before any change)."""
-        host = position.cpu()
-        wanted = torch.arange(start, start + host.numel(), dtype=host.dtype)
+    def _position_mismatch(self, position: torch.Tensor, start: int) -> None:
+        """Compares GPU positions with start, start + 1, ... on the device; a
+        mismatch raises the flag word that the next flag read reports."""
+        flags = self._flag_words(position.device)
+        nat.check(nat.lib().iq_check_positions(
+            position.data_ptr(), position.element_size(), position.stride(0), position.numel(), start,
+            flags.data_ptr() + 4 * _POSITION_BAD, nat.stream_handle(position.device)))
+
+    def _position_check(self, position: torch.Tensor, start: int) -> None:
+        """Synchronous comparison with start, start + 1, ... (raises before any
+        change), a mismatch still pending from an earlier step included."""
         flags = self._flags
-        deferred = flags is not None and bool(flags[_POSITION_BAD].item())
-        if deferred:
-            flags[_POSITION_BAD].zero_()
-        if deferred or not bool((host == wanted).all()):
+        if position.is_cuda and (flags is None or flags.device == position.device):
+            self._position_mismatch(position, start)
+            bad = bool(self._flags.tolist()[_POSITION_BAD])
+        else:
+            host = position.cpu()
+            bad = not bool((host == torch.arange(start, start + host.numel(), dtype=host.dtype)).all())
+            bad = (flags is not None and bool(flags[_POSITION_BAD].item())) or bad
+        if bad:
+            if self._flags is not None:
+                self._flags[_POSITION_BAD].zero_()
             self._position_checked = None
             raise ValueError(_POSITION_ERROR)
 
@@ -536,7 +558,10 @@ class InQuantCache(_HFCache):
         layer, position = self._check(key_states, value_states, layer_idx, cache_kwargs)
         start = 0 if layer is None else layer.seq_length
         if position is not None:
-            self._host_position_check(position, start)
+            if position.device == key_states.device and position.is_cuda and self._seals(layer, key_states.shape[2]):
+                self._position_mismatch(position, start)      # read with the encoders' flags, before any change
+            else:
+                self._position_check(position, start)
         if layer is None:
             layer = _LayerCache(key_states.shape, key_states.dtype, key_states.device)
             result = (key_states, value_states)
@@ -571,7 +596,7 @@ class InQuantCache(_HFCache):
 
     def _append_general(self, layer, key_states, value_states, position, blocks) -> PackedAttentionView:
         if position is not None:
-            self._host_position_check(position, layer.seq_length)
+            self._position_check(position, layer.seq_length)
         sink = (layer.sink_key, layer.sink_value)
         before = (layer.residual_key, layer.residual_value)
         pending_k = key_states if before[0] is None else torch.cat((before[0], key_states), 2)
@@ -593,7 +618,7 @@ class InQuantCache(_HFCache):
         pos_ptr, pos_bytes = None, 0
         if position is not None:
             if position.device.type != "cuda":
-                self._host_position_check(position, layer.seq_length)
+                self._position_check(position, layer.seq_length)
             else:
                 pos_ptr, pos_bytes = position.data_ptr(), position.element_size()
                 # a position tensor already verified against this start, and not
@@ -691,12 +716,20 @@ class InQuantCache(_HFCache):
             raise ValueError(_BAD_K)
         if bad_value:
             raise ValueError(value_error)
-        layer.runs.append((len(layer.key_blocks), len(layer.key_blocks) + len(new_keys)))
-        layer.key_blocks.extend(new_keys)
-        layer.value_blocks.extend(new_values)
+        have = layer.block_count
+        layer.runs.append((have, have + count))
+        layer.batches.append((new_keys, new_values))
         layer.block_tuples = None
         if cfg.track_peak_bytes:
-            layer.packed_nbytes += sum(b.nbytes for b in new_keys) + sum(b.nbytes for b in new_values)
+            layer.packed_nbytes += new_keys.nbytes + new_values.nbytes
+
+    def _seals(self, layer: _LayerCache | None, tokens: int) -> int:
+        """Blocks that appending ``tokens`` to the layer (None: a new one) seals."""
+        cfg = self.config
+        have = 0 if layer is None or layer.sink is None else layer.sink.count
+        live = 0 if layer is None or layer.tail is None else layer.tail.count
+        rest = tokens - max(0, min(cfg.sink_tokens - have, tokens))
+        return max(0, (live + rest - cfg.residual_length) // cfg.block_size)
 
     def _ingest(self, layer: _LayerCache, keys, values) -> None:
         """General append of any number of tokens (cache.py:271-306 semantics)."""
@@ -714,7 +747,7 @@ class InQuantCache(_HFCache):
         m = n - take
         tail = layer.tail
         live = 0 if tail is None else tail.count
-        blocks = max(0, (live + m - cfg.residual_length) // cfg.block_size)
+        blocks = self._seals(layer, n)
         if blocks:
             pending_k = rest_k if not live else torch.cat((tail.keys(), rest_k), 2)
             pending_v = rest_v if not live else torch.cat((tail.values(), rest_v), 2)
@@ -778,18 +811,16 @@ class InQuantCache(_HFCache):
         sink_n = 0 if layer.sink is None else layer.sink.count
         tail_n = 0 if layer.tail is None else layer.tail.count
         new_n = 0 if new_keys is None else new_keys.shape[2]
-        packed = sum(b.shape[2] for b in layer.key_blocks)
-        total = sink_n + packed + tail_n + new_n
+        total = sink_n + layer.block_count * self.config.block_size + tail_n + new_n
         out, pairs = [], []
-        for side, blocks in ((0, layer.key_blocks), (1, layer.value_blocks)):
+        for side in (0, 1):
             dense = torch.empty((1, heads, total, dim), dtype=layer.dtype, device=layer.device)
             if sink_n:
                 pairs.append((layer.sink.values() if side else layer.sink.keys(), dense[:, :, :sink_n]))
             at = sink_n
-            for i, j in layer.runs:
-                run = _run_block(blocks, i, j)                           # [n, H, T, D]
-                _dequantize_into(run, dense, at)
-                at += (j - i) * run.shape[2]
+            for batch in layer.batches:
+                _dequantize_into(batch[side], dense, at)
+                at += batch[side].shape[0] * batch[side].shape[2]
             if tail_n:
                 pairs.append((layer.tail.values() if side else layer.tail.keys(), dense[:, :, at:at + tail_n]))
             if new_n:
@@ -802,8 +833,8 @@ class InQuantCache(_HFCache):
     # ------------------------------------------------------------ accounting (cache.py:346-394)
     def _blocks(self):
         for layer in self._layers.values():
-            yield from layer.key_blocks
-            yield from layer.value_blocks
+            for batch in layer.batches:
+                yield from batch
 
     @property
     def payload_nbytes(self) -> int:
@@ -847,7 +878,7 @@ class InQuantCache(_HFCache):
             "sink_nbytes": self.sink_nbytes,
             "auxiliary_nbytes": self.auxiliary_nbytes,
             "bf16_nbytes": dense,
-            "quantized_layer_tokens": sum(b.shape[2] for l in self._layers.values() for b in l.key_blocks),
+            "quantized_layer_tokens": sum(l.block_count for l in self._layers.values()) * self.config.block_size,
             "kv_reduction_vs_bf16": (1 - total / dense) if dense else 0.0,
             # preallocated dense rows not yet holding tokens (not part of nbytes)
             "dense_reserve_nbytes": sum(l.reserved_nbytes() for l in self._layers.values()),

@@ -98,15 +98,10 @@ def quantize_value_blocks(tensor: torch.Tensor, block_count: int, block_size: in
     """Encode the first `block_count` temporal blocks of [1, H, T, D] with
     statistics per (block, head) (value_codec.py:75-88): one launch over the
     strided [blocks, H, B, D] view, one PackedValues view per block."""
-    return _value_blocks(tensor, block_count, block_size, bits, group_size, None)
-
-
-def _value_blocks(tensor, block_count, block_size, bits, group_size, bad):
-    """quantize_value_blocks with the private non-finite flag of quantize_values."""
     if not block_count:
         return []
     _, heads, _, dim = tensor.shape
     blocked = tensor[0, :, :block_count * block_size].unflatten(1, (block_count, block_size)).transpose(0, 1)
-    packed = quantize_values(blocked, bits, group_size, _flag=bad)
+    packed = quantize_values(blocked, bits, group_size)
     return _per_block(packed, block_count, (1, heads, block_size, dim), PackedValues, bits=bits,
                       group_size=group_size)

@@ -47,3 +47,24 @@ def test_copied_rows(offset, width):
     _copy_rows([(a, dst[:, :, 25:45, :width]), (b, dst[:, :, :17, :width]), (a[:, :, :0], dst[:, :, :0, :width])])
     assert torch.equal(dst[:, :, 25:45, :width], a) and torch.equal(dst[:, :, :17, :width], b)
     assert np.count_nonzero(dst.float().cpu().numpy()) <= 3 * 37 * width
+
+
+@pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
+def test_positions_are_checked_before_a_sealing_update_changes_the_layer(dtype):
+    from inquant.cache import CacheConfig, InQuantCache
+    cache = InQuantCache(CacheConfig(block_size=8, residual_length=4, sink_tokens=2, value_bits=2))
+    k = torch.randn(1, 2, 70, 64, device="cuda").bfloat16()
+    pos = torch.arange(140, dtype=dtype, device="cuda")[::2] // 2               # a strided view
+    wrong = pos.clone()
+    wrong[30] += 1
+    cache.update(k[:, :, :20], k[:, :, :20], 0, {"cache_position": pos[:20]})
+    before, blocks = cache.materialize(0), list(cache._layers[0].key_blocks)
+    for bad in (wrong[20:60], pos[21:61]):
+        with pytest.raises(ValueError, match="contiguous append"):
+            cache.update(k[:, :, 20:60], k[:, :, 20:60], 0, {"cache_position": bad})
+        assert cache.get_seq_length() == 20 and len(cache._layers[0].key_blocks) == len(blocks)
+        assert all(torch.equal(a, b) for a, b in zip(cache.materialize(0), before))
+    cache.update(k[:, :, 20:60], k[:, :, 20:60], 0, {"cache_position": pos[20:60]})
+    assert cache.get_seq_length() == 60 and cache._layers[0].key_blocks[0] is blocks[0]
+    with pytest.raises(ValueError, match="contiguous append"):
+        InQuantCache(cache.config).update(k, k, 0, {"cache_position": wrong})
