@@ -1007,12 +1007,11 @@ __global__ __launch_bounds__(K4_THREADS) void k4_quantize_rows(K4Args a, int64_t
 // channel-contiguous rows.  The block streams through LDS in 32-token chunks
 // (double-buffered, 16-byte loads, three chunks in flight while the current
 // one is consumed), twice:
-//   pass 1  waves 0-1: the fp64 Welford var_mean of channel tid (min_error
-//           only); delta / n uses a table of RN(1/n) and one remainder fma,
-//           which is the correctly rounded quotient for n <= 256 (sealed
-//           blocks: one fma with compile-time constants, see step_c);
-//           waves 2-3: sampled sums (torch cascade order), amax and
-//           finiteness as an integer max of the 16-bit magnitudes;
+//   pass 1  thread (half, channel) sums x and x^2 of every other token in
+//           fp64 (min_error only) and takes amax and finiteness as an integer
+//           max of the 16-bit magnitudes; one half also adds the sampled
+//           sums (torch cascade order).  The donor errors come from the sums
+//           with a certificate (k4_stats_dev.h);
 //   then    donor selection by the whole workgroup (iq_select_tile128);
 //           the sequential donor picks run on one wavefront alone, and with a
 //           value row to encode (page mode, or VB = 2 / 4) the other three
@@ -1020,8 +1019,13 @@ __global__ __launch_bounds__(K4_THREADS) void k4_quantize_rows(K4Args a, int64_t
 //           v_encode_rows), reading them from HBM while it is otherwise idle;
 //   pass 2  every thread quantizes 8 channels of a token per step, writing
 //           4 payload bytes.
+// With a sequential fp64 Welford chain per channel on two of the wavefronts
+// (they waited for each other at every chunk) a layer of 32768 tokens x 8
+// heads took 82 us with K4 keys and values and 58-62 with 2-bit values; with
+// the sums on all four 76-78 and 57-58, and 32768 tokens x 4 heads in
+// 256-token pages 38.9 instead of 42.3.
 // LDS stays under 40 KiB, so four blocks share a compute unit and their
-// latency-bound phases (the Welford chains, the donor picks) overlap.
+// latency-bound phases (the chunk waits, the donor picks) overlap.
 // Bit-identical to k4_encode_kernel.
 constexpr int TILE_D = 128;
 constexpr int TILE_T = 256;
@@ -1081,8 +1085,7 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     constexpr int ROWLEN = DMA ? TILE_D : XROW;       // u16 per staged row
     static_assert(!DMA || (NBUF >= 2 && NBUF <= 4), "chunk buffers");
     __shared__ __attribute__((aligned(16))) uint16_t s_x[NBUF][CH * ROWLEN];
-    __shared__ double s_rcp[TILE_T];    // RN(1 / n), n = 1 .. T
-    __shared__ __attribute__((aligned(16))) float s_sal[TILE_D], s_smean[TILE_D], s_err[TILE_D], s_amax[TILE_D],
+    __shared__ __attribute__((aligned(16))) float s_sal[TILE_D], s_smean[TILE_D], s_err[TILE_D], s_ehi[TILE_D], s_amax[TILE_D],
         s_scale[TILE_D];
     __shared__ int16_t s_src_of[TILE_D];
     __shared__ uint8_t s_is_src[TILE_D];
@@ -1091,7 +1094,7 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     __shared__ __attribute__((aligned(16))) int s_part[K4_THREADS];
     __shared__ __attribute__((aligned(16))) uint8_t s_flag[TILE_D];
     __shared__ int16_t s_list[TILE_D / 2];
-    __shared__ int s_bad;
+    __shared__ int s_bad, s_again;
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int64_t row = b * a.H + h;
@@ -1168,7 +1171,8 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     // visits chunks in order, chunk ch in buf_of(ch) during body(ch)
     auto stream = [&](auto &&body) {
         if constexpr (DMA) {
-#pragma unroll
+            // rolled: unrolled, the statistics spill 38 registers
+#pragma unroll 1
             for (int ch = 0; ch < NCH; ++ch) {
                 // requested so far: chunks 0 .. ch + NBUF - 2
                 wait_chunk_barrier(min(NBUF - 2, NCH - 1 - ch));
@@ -1193,21 +1197,17 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     };
 
     start_stream();
-    if (NCH == 0 && tid < T) s_rcp[tid] = 1.0 / (double)(tid + 1);
     if (tid == 0) s_bad = 0;
     if constexpr (!DMA) store_chunk(seg[0], 0);
     __syncthreads();
 
-    // ---- pass 1: statistics.  Two waves run the Welford chains (channel
-    // tid & 127) and two the sums; which pair does which alternates between
-    // neighbouring blocks, so that the blocks sharing a compute unit spread
-    // the fp64 chains over all four SIMDs instead of stacking them on two.
-    const bool welford = ((tid >> 7) ^ ((lin >> 8) & 1)) == 0;
-    // The Welford chains are the critical path of pass 1 (the sums waves
-    // then wait at every chunk barrier), so their waves issue first.
-    if (welford && a.min_error) __builtin_amdgcn_s_setprio(2);
-    double mean = 0.0, m2 = 0.0;                  // Welford waves
-    IqCascade sa, sm;                             // sums waves
+    // ---- pass 1: statistics.  Thread (half, channel c1) takes the tokens of
+    // one parity; which wavefronts are half 1, and add the samples as well,
+    // alternates between the blocks that share a compute unit.
+    const int half = (tid >> 7) ^ ((lin >> 8) & 1);
+    double *const s_sum1 = (double *)s_key, *const s_sum2 = (double *)s_part;     // half 1's sums, until the selection
+    double sum1 = 0.0, sum2 = 0.0;
+    IqCascade sa, sm;                             // half 1
     sa.init(ns);
     sm.init(ns);
     uint32_t amax_bits = 0;
@@ -1216,92 +1216,26 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     stream([&](int ch) {
         const uint16_t *xs = buf_of(ch) + c1;
         const int t0 = ch * CH, nt = min(CH, T - t0);
-        if (welford) {
+        // |x| as 16-bit integers: for finite values their order is the
+        // order of the magnitudes, and inf / NaN sort above every finite one
+        auto take = [&](uint32_t u) {
+            amax_bits = max(amax_bits, u & 0x7fffu);
             if (a.min_error) {
-                auto step = [&](float xf, double y, int t) {
-                    const double dv = (double)xf;
-                    const double delta = __dsub_rn(dv, mean);
-                    const double q0 = __dmul_rn(delta, y);
-                    const double r = __builtin_fma(-q0, (double)(t + 1), delta);
-                    mean = __dadd_rn(mean, __builtin_fma(r, y, q0));
-                    const double nd = __dsub_rn(dv, mean);
-                    m2 = __dadd_rn(m2, __dmul_rn(delta, nd));
-                };
-                // A sealed block's counts n = t + 1 are compile-time constants, and
-                // so are y_hi = RN(1/n) and y_lo = RN((1 - y_hi n) / n) (the residual
-                // 1 - y_hi n is exact).  delta / n is then one fma:
-                // RN(delta y_hi + RN(delta y_lo)).  A quotient by an integer n <= 256
-                // is never a midpoint between doubles and lies at least ulp / 512
-                // from one (its odd part would need 54 bits), while
-                // delta y_hi + RN(delta y_lo) is within 2^-105 |delta / n|, i.e.
-                // 2^-52 ulp, of it: the fma returns the correctly rounded quotient,
-                // with one dependent operation fewer than the remainder correction.
-                auto step_c = [&](float xf, int t) {
-                    const double n = (double)(t + 1);
-                    double yh = 1.0 / n;
-                    double yl = __builtin_fma(-yh, n, 1.0) / n;
-                    asm("" : "+s"(yh), "+s"(yl));      // scalar operands of the mul and the fma
-                    const double dv = (double)xf;
-                    const double delta = __dsub_rn(dv, mean);
-                    mean = __dadd_rn(mean, __builtin_fma(delta, yh, __dmul_rn(delta, yl)));
-                    const double nd = __dsub_rn(dv, mean);
-                    m2 = __dadd_rn(m2, __dmul_rn(delta, nd));
-                };
-                if constexpr (NCH > 0) {
-                    // LDS reads of the next eight tokens in flight while the
-                    // current eight dependent steps run
-                    float cur[8], nxt[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) cur[u] = tile_f32<F16IN>(xs[u * ROWLEN]);
-#pragma unroll
-                    for (int g = 0; g < CH; g += 8) {
-                        const int gn = g + 8 < CH ? g + 8 : g;
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) nxt[u] = tile_f32<F16IN>(xs[(gn + u) * ROWLEN]);
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) step_c(cur[u], t0 + g + u);
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) cur[u] = nxt[u];
-                    }
-                } else if (nt == CH) {
-                    // LDS reads of the next eight tokens in flight while the
-                    // current eight dependent steps run
-                    float cur[8], nxt[8];
-                    double ycur[8], ynxt[8];
-#pragma unroll
-                    for (int u = 0; u < 8; ++u) {
-                        cur[u] = tile_f32<F16IN>(xs[u * ROWLEN]);
-                        ycur[u] = s_rcp[t0 + u];
-                    }
-#pragma unroll
-                    for (int g = 0; g < CH; g += 8) {
-                        const int gn = g + 8 < CH ? g + 8 : g;
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) {
-                            nxt[u] = tile_f32<F16IN>(xs[(gn + u) * ROWLEN]);
-                            ynxt[u] = s_rcp[t0 + gn + u];
-                        }
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) step(cur[u], ycur[u], t0 + g + u);
-#pragma unroll
-                        for (int u = 0; u < 8; ++u) {
-                            cur[u] = nxt[u];
-                            ycur[u] = ynxt[u];
-                        }
-                    }
-                } else {
-                    for (int u = 0; u < nt; ++u) step(tile_f32<F16IN>(xs[u * ROWLEN]), s_rcp[t0 + u], t0 + u);
-                }
+                const double d = (double)tile_f32<F16IN>(u);
+                sum1 = __dadd_rn(sum1, d);
+                sum2 = __builtin_fma(d, d, sum2);
             }
+        };
+        if (nt == CH) {
+            uint32_t u[CH / 2];
+#pragma unroll
+            for (int k = 0; k < CH / 2; ++k) u[k] = xs[(2 * k + half) * ROWLEN];
+#pragma unroll
+            for (int k = 0; k < CH / 2; ++k) take(u[k]);
         } else {
-            // |x| as 16-bit integers: for finite values their order is the
-            // order of the magnitudes, and inf / NaN sort above every finite one
-            if (nt == CH) {
-#pragma unroll
-                for (int u = 0; u < CH; ++u) amax_bits = max(amax_bits, (uint32_t)xs[u * ROWLEN] & 0x7fffu);
-            } else {
-                for (int u = 0; u < nt; ++u) amax_bits = max(amax_bits, (uint32_t)xs[u * ROWLEN] & 0x7fffu);
-            }
+            for (int k = half; k < nt; k += 2) take(xs[k * ROWLEN]);
+        }
+        if (half) {
             // the samples r * stride that fall in this chunk, in order
             for (; next_sample < t0 + nt; next_sample += stride) {
                 const float v = tile_f32<F16IN>(xs[(next_sample - t0) * ROWLEN]);
@@ -1310,17 +1244,12 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
             }
         }
     });
-    if (welford) {
-        if (a.min_error) {
-            s_err[c1] = (float)(m2 / (double)T);      // var; the mean term is added below
-            s_smean[c1] = (float)mean;                // full mean, replaced below
-        }
-    } else {
-        s_amax[c1] = tile_f32<F16IN>(amax_bits);
+    if (half) {
+        s_sum1[c1] = sum1;
+        s_sum2[c1] = sum2;
+        s_amax[c1] = __uint_as_float(amax_bits);
         s_sal[c1] = sa.finish() / (float)ns;
-        if (amax_bits >= (F16IN ? 0x7c00u : 0x7f80u)) s_bad = 1;     // an inf or NaN in the channel
-        // stash the sampled mean until the Welford waves are done with s_smean
-        s_scale[c1] = sm.finish() / (float)ns;
+        s_smean[c1] = sm.finish() / (float)ns;
     }
     // A sealed block's last NBUF chunks are still in the buffers after pass 1
     // and pass 2 quantizes them first (RESIDENT), reloading the others into
@@ -1385,13 +1314,17 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
         }
     }
 
-    if (tid < TILE_D) {
-        const float smean = s_scale[tid];
+    if (!half) {
+        amax_bits = max(amax_bits, __float_as_uint(s_amax[c1]));
+        const float amax = tile_f32<F16IN>(amax_bits);
+        s_amax[c1] = amax;
+        if (amax_bits >= (F16IN ? 0x7c00u : 0x7f80u)) s_bad = 1;     // an inf or NaN in the channel
         if (a.min_error) {
-            const float diff = __fsub_rn(s_smean[tid], smean);
-            s_err[tid] = __fadd_rn(s_err[tid], __fmul_rn(diff, diff));
+            const IqErrRange r =
+                iq_err_range(__dadd_rn(sum1, s_sum1[c1]), __dadd_rn(sum2, s_sum2[c1]), amax, s_smean[c1], T);
+            s_err[c1] = r.lo;
+            s_ehi[c1] = r.hi;
         }
-        s_smean[tid] = smean;
     }
     __syncthreads();
 
@@ -1400,6 +1333,11 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     else __builtin_amdgcn_s_setprio(0);
     iq_select_tile128(s_sal, a.min_error ? s_err : nullptr, (int)a.count, s_src, s_don, s_is_src, s_src_of,
                       s_key, s_part, s_flag, s_list, vtid);
+    if (vwave == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        const bool again = a.min_error && !s_bad && !iq_pool_certain(s_err, s_ehi, TILE_D, s_is_src, s_src_of);
+        if (lane == 0) s_again = again;
+    }
     if constexpr (VBITS > 0) {
         if (vwave > 0) {
             bool vbad = false;
@@ -1421,6 +1359,24 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     }
     __builtin_amdgcn_s_setprio(1);
     __syncthreads();
+    if (__builtin_expect(s_again, 0)) {
+        // the pool is uncertain: the reference's sequential errors, and the selection on them
+        if (tid < TILE_D) {
+            double mean = 0.0, m2 = 0.0;
+#pragma unroll 1
+            for (int t = 0; t < T; ++t) {
+                const double dv = (double)tile_f32<F16IN>(xr[(int64_t)t * a.st + tid]);
+                const double delta = __dsub_rn(dv, mean);
+                mean = __dadd_rn(mean, delta / (double)(t + 1));
+                m2 = __dadd_rn(m2, __dmul_rn(delta, __dsub_rn(dv, mean)));
+            }
+            const float diff = __fsub_rn((float)mean, s_smean[tid]);
+            s_err[tid] = __fadd_rn((float)(m2 / (double)T), __fmul_rn(diff, diff));
+        }
+        __syncthreads();
+        if (tid < 64) iq_select_wave128(s_sal, s_err, (int)a.count, s_src, s_don, s_is_src, s_src_of, s_list);
+        __syncthreads();
+    }
 
     const float flt_min = 1.17549435e-38f;
     if (tid < TILE_D) {

@@ -126,3 +126,23 @@ def test_pool_picks(D, count):
     got = _reuse_map(torch.from_numpy(sal).cuda(), count, torch.from_numpy(err).cuda())
     for a, b in zip(got, want):
         np.testing.assert_array_equal(a.cpu().numpy(), b)
+
+
+# the tile encoder's certificate: tied and equal channels in blocks of 128 16-bit channels (whole, ragged, paged)
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [256, 100, 33])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_blocks_with_tied_errors(T, dtype):
+    x = synth.normal(T, (2, 3, T, 128))
+    x[0, 0, :, 8:] = x[0, 0, :, 8:9]                    # 120 equal channels
+    x[0, 1, :, 20:90] = np.arange(20, 90) / 7.0         # 70 constant channels
+    x[0, 2, :, 4:120] = x[0, 2, :, 4:5]                 # equal but for the tokens' order
+    x[0, 2, :, 5:120:2] = x[0, 2, ::-1, 5:120:2]
+    x[1, 0, :, 30:] = 0
+    _check(torch.from_numpy(x).cuda().to(dtype), 8, 0.125, "min_error")
+    if T == 256:
+        from inquant_vllm.layout import PageLayout, pack_pages
+        xt = torch.from_numpy(x).cuda().to(dtype)
+        f = xt.float().cpu().numpy()
+        want = oracle.pack_pages(oracle.k4_quantize(f, 8, 0.125, "min_error"), oracle.v_quantize(f, 2, 64), 3, T)
+        np.testing.assert_array_equal(pack_pages(xt, xt, PageLayout(T, 3)).cpu().numpy(), want)
