@@ -46,7 +46,7 @@ struct PrefillArgs {
     void *out;
     int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;   // element strides (token, head)
     const int32_t *cu;                                        // [n_seq + 1] token offsets
-    int tiles, Hq;                                            // query tiles per sequence, query heads
+    int tiles, span, n_seq, Hq;                               // query tiles per sequence, places per group, sequences, query heads
     int G;
     float c_log2;                                             // softmax scale * log2(e)
     int odt;
@@ -107,19 +107,26 @@ __global__ __launch_bounds__(NT, 2) void prefill_attn(PrefillArgs a)
     __shared__ PrefillSmem sm;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int c32 = lane & 31, h32 = lane >> 5;
-    // Workgroup i of a sequence's slice runs on XCD i % 8 (the dispatcher
-    // deals workgroups round-robin over the eight XCDs; every slice is a
-    // multiple of 8 long).  Each XCD takes a contiguous range of the slice's
-    // (query head, query tile) items, so the workgroups resident on it read
-    // the K/V of one or two KV heads and find them in its own L2 (8K causal
-    // Qwen2.5-7B: 713 -> 577 us against items dealt out in grid order).
-    // Within a query head, tiles go longest first.
-    const int per = (a.tiles * a.Hq + 7) / 8;
-    const int item = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3);
-    if (item >= a.tiles * a.Hq) return;          // the slice's padding
-    const int hq = item / a.tiles, seq = blockIdx.y, h = hq / a.G;
+    // Workgroup i runs on XCD i % 8 (the dispatcher deals workgroups
+    // round-robin over the eight XCDs).  An item is a (query tile, sequence,
+    // query head); its cost grows with the tile's place in its sequence alone.
+    // Tiles go from the last places to the first, over all sequences, so the
+    // longest items start first and the last to run are short; of each group
+    // of `span` places an XCD takes the same share of neighbouring heads in
+    // every sequence (span Hq / 8 items), so the work of the XCDs is even and
+    // an XCD's resident workgroups read the K/V of a KV head at about the same
+    // time, out of its own L2.  8K causal, 28 query heads: 516 us (933 TFLOP/s)
+    // with a contiguous range of (head, tile) items per XCD, where four of the
+    // XCDs had 15% more work than the others and ended on long tiles, 468 (1028)
+    // with these; seven prompts of up to 4.1K tokens, 32 heads: 293 and 281.
+    const int share = a.span * a.Hq / 8;
+    const int j = (int)(blockIdx.x >> 3), rest = j % (a.n_seq * share);
+    const int at = (int)(blockIdx.x & 7) * share + rest % share;
+    const int seq = rest / share, hq = at / a.span, h = hq / a.G;
+    const int place = a.tiles - 1 - (j / (a.n_seq * share) * a.span + at % a.span);
+    if (place < 0) return;                       // the last group's padding
     const int start = a.cu[seq], len = a.cu[seq + 1] - start;
-    const int q0 = (a.tiles - 1 - item % a.tiles) * QT;
+    const int q0 = place * QT;
     if (q0 >= len) return;                       // uniform: no barrier is skipped by part of the group
     const int qw = q0 + QW * wave;               // this wavefront's first query
     const int my_q = qw + c32;                   // the query of this lane's column
@@ -318,15 +325,21 @@ extern "C" int iq_prefill_attention(const void *q, const void *k, const void *v,
     const int64_t obytes = out_dtype == IQ_F32 ? 4 : 2;
     const int vec_out = (uintptr_t)out % (4 * obytes) == 0 && o_st % 4 == 0 && o_sh % 4 == 0;
     const int64_t tiles = (max_seqlen + QT - 1) / QT;
-    // one slice of workgroups per sequence, padded to a multiple of 8
-    const int64_t slice = (tiles * Hq + 7) / 8 * 8;
-    IQ_CHECK_ARG(slice <= 0x7fffffffLL, "iq_prefill_attention: too many query tiles");
-    PrefillArgs a{(const uint16_t *)q, (const uint16_t *)k, (const uint16_t *)v, out, q_st, q_sh, k_st, k_sh,
-                  v_st, v_sh, o_st, o_sh, cu_seqlens, (int)tiles, (int)Hq, (int)(Hq / H),
-                  scale * 1.44269504088896341f, out_dtype, vec_out};
-    const dim3 grid((unsigned)slice, (unsigned)n_seq), block(NT);
-    if (dtype == IQ_F16) hipLaunchKernelGGL(prefill_attn<true>, grid, block, 0, (hipStream_t)stream, a);
-    else hipLaunchKernelGGL(prefill_attn<false>, grid, block, 0, (hipStream_t)stream, a);
+    // places per group: the least number for which the XCDs' shares are whole
+    int64_t span = 1;
+    while (span * Hq % 8) span *= 2;
+    const int64_t per_seq = (tiles + span - 1) / span * span * Hq;
+    constexpr int64_t MOST = 0xffffffffLL / NT;          // workgroups of a launch (2^32 threads)
+    IQ_CHECK_ARG(per_seq <= MOST, "iq_prefill_attention: too many query tiles");
+    for (int64_t s0 = 0; s0 < n_seq; s0 += MOST / per_seq) {
+        const int64_t n = n_seq - s0 < MOST / per_seq ? n_seq - s0 : MOST / per_seq;
+        PrefillArgs a{(const uint16_t *)q, (const uint16_t *)k, (const uint16_t *)v, out, q_st, q_sh, k_st, k_sh,
+                      v_st, v_sh, o_st, o_sh, cu_seqlens + s0, (int)tiles, (int)span, (int)n, (int)Hq, (int)(Hq / H),
+                      scale * 1.44269504088896341f, out_dtype, vec_out};
+        const dim3 grid((unsigned)(per_seq * n)), block(NT);
+        if (dtype == IQ_F16) hipLaunchKernelGGL(prefill_attn<true>, grid, block, 0, (hipStream_t)stream, a);
+        else hipLaunchKernelGGL(prefill_attn<false>, grid, block, 0, (hipStream_t)stream, a);
+    }
     IQ_CHECK_LAUNCH("prefill_attn");
     return IQ_OK;
 }
