@@ -1,12 +1,12 @@
 // K4 neighbor-slot encoder and standalone donor selector (gfx950).
 //
-// One 256-thread workgroup encodes one (batch, head) row of x[B, H, T, D]:
-//   phase 1  per-channel statistics: sampled saliency and mean in torch's
-//            CPU summation order, full-block amax, and for min_error the
-//            fp64 Welford var_mean (codec.py:200-210);
-//   phase 2  donor selection by wavefront 0 (select_dev.h);
-//   phase 3  scales, 4-bit slots, 8-bit salient codes split across the
-//            source and donor slots, nibble packing, padding (codec.py:218-233).
+// A (batch, head) row of x[B, H, T, D] goes through
+//   1  per-channel statistics: sampled saliency and mean in torch's CPU
+//      summation order, full-row amax, and for min_error the donor error
+//      (codec.py:200-210);
+//   2  donor selection (select_dev.h);
+//   3  scales, 4-bit slots, 8-bit salient codes split across the source and
+//      donor slots, nibble packing, padding (codec.py:218-233).
 // Results are bit-identical to the reference CPU implementation.
 #include "k4_stats_dev.h"
 #include "select_dev.h"
@@ -1541,8 +1541,12 @@ __global__ __launch_bounds__(K4_THREADS) void k4_encode_page_rows(K4Args a, int6
 #pragma unroll
     for (int t = 0; t < T; ++t) {
         const uint32_t w = *(const uint32_t *)(xs + t * ROW + 2 * lane);
-        // delta / n as in the tile encoder's step_c: one fma with the
-        // compile-time pair RN(1/n), RN((1 - RN(1/n) n) / n)
+        // delta / n with y_hi = RN(1/n) and y_lo = RN((1 - y_hi n) / n) (the
+        // residual 1 - y_hi n is exact) is one fma: RN(delta y_hi +
+        // RN(delta y_lo)).  A quotient by an integer n <= 256 is never a
+        // midpoint between doubles and lies at least ulp / 512 from one, while
+        // the fma's exact argument is within 2^-52 ulp of it
+        // (tests/test_welford_division.py)
         const double n = (double)(t + 1);
         const double yh = 1.0 / n;
         const double yl = __builtin_fma(-yh, n, 1.0) / n;

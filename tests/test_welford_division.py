@@ -1,5 +1,5 @@
-"""The quotient identity of the tile encoder's Welford step for sealed blocks
-(csrc/k4_encode.hip, step_c): for integers 1 <= n <= 256 and finite doubles
+"""The quotient identity of the page row encoder's Welford step
+(csrc/k4_encode.hip, k4_encode_page_rows): for integers 1 <= n <= 256 and finite doubles
 delta, RN(delta / n) == fma(delta, y_hi, RN(delta * y_lo)) with
 y_hi = RN(1 / n) and y_lo = RN(fma(-y_hi, n, 1) / n).  The torch CPU
 var_mean that the encoder restates divides by n once per step
