@@ -108,11 +108,18 @@ class PackedAttentionView(NamedTuple):
     seq_length: int
 
 
+def _launches(tensor: torch.Tensor) -> bool:
+    """Whether a launch on the tensor's stream runs on its GPU: the default
+    stream's handle names the current device's, so tensors of another one (a
+    model spread over GPUs) are left to torch, which switches devices."""
+    return tensor.is_cuda and tensor.device.index == torch.cuda.current_device()
+
+
 def _copy_rows(pairs) -> None:
     """Copies (source, destination) pairs of [1, H, n, D] views, at most eight
     and of one head count, width and dtype, in one launch."""
     first = pairs[0][0]
-    if not first.is_cuda or any(s.stride(3) != 1 or d.stride(3) != 1 for s, d in pairs):
+    if not _launches(first) or any(s.stride(3) != 1 or d.stride(3) != 1 for s, d in pairs):
         for s, d in pairs:
             d.copy_(s)
         return
@@ -537,7 +544,7 @@ class InQuantCache(_HFCache):
         """Synchronous comparison with start, start + 1, ... (raises before any
         change), a mismatch still pending from an earlier step included."""
         flags = self._flags
-        if position.is_cuda and (flags is None or flags.device == position.device):
+        if _launches(position) and (flags is None or flags.device == position.device):
             self._position_mismatch(position, start)
             bad = bool(self._flags.tolist()[_POSITION_BAD])
         else:
@@ -558,7 +565,7 @@ class InQuantCache(_HFCache):
         layer, position = self._check(key_states, value_states, layer_idx, cache_kwargs)
         start = 0 if layer is None else layer.seq_length
         if position is not None:
-            if position.device == key_states.device and position.is_cuda and self._seals(layer, key_states.shape[2]):
+            if position.device == key_states.device and _launches(position) and self._seals(layer, key_states.shape[2]):
                 self._position_mismatch(position, start)      # read with the encoders' flags, before any change
             else:
                 self._position_check(position, start)

@@ -49,6 +49,20 @@ def test_copied_rows(offset, width):
     assert np.count_nonzero(dst.float().cpu().numpy()) <= 3 * 37 * width
 
 
+def test_rows_and_positions_of_another_device_are_left_to_torch(monkeypatch):
+    from inquant.cache import CacheConfig, InQuantCache
+    k = torch.randn(1, 2, 9, 64, device="cuda").bfloat16()
+    pos = torch.arange(9, device="cuda")
+    cache = InQuantCache(CacheConfig(block_size=8, residual_length=4, sink_tokens=2))
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)                # as under torch.cuda.device(1)
+    monkeypatch.setattr("inquant.cache.nat.lib", lambda: pytest.fail("launched on the current device"))
+    cache.update(k[:, :, :7], k[:, :, :7], 0, {"cache_position": pos[:7]})
+    with pytest.raises(ValueError, match="contiguous append"):
+        cache.update(k[:, :, 7:], k[:, :, 7:], 0, {"cache_position": pos[6:8]})
+    for got in cache.update(k[:, :, 7:], k[:, :, 7:], 0, {"cache_position": pos[7:]}):
+        assert torch.equal(got, k)
+
+
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
 def test_positions_are_checked_before_a_sealing_update_changes_the_layer(dtype):
     from inquant.cache import CacheConfig, InQuantCache
