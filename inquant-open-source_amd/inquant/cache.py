@@ -564,17 +564,27 @@ class InQuantCache(_HFCache):
         on the first call, else dequantized history ++ the new tokens)."""
         layer, position = self._check(key_states, value_states, layer_idx, cache_kwargs)
         start = 0 if layer is None else layer.seq_length
-        if position is not None:
-            if position.device == key_states.device and _launches(position) and self._seals(layer, key_states.shape[2]):
-                self._position_mismatch(position, start)      # read with the encoders' flags, before any change
+        deferred = (position is not None and position.device == key_states.device and _launches(position)
+                    and self._seals(layer, key_states.shape[2]) > 0)
+        if deferred:
+            self._position_mismatch(position, start)      # read with the encoders' flags, before any change
+        elif position is not None:
+            self._position_check(position, start)
+        try:
+            if layer is None:
+                layer = _LayerCache(key_states.shape, key_states.dtype, key_states.device)
+                result = (key_states, value_states)
             else:
-                self._position_check(position, start)
-        if layer is None:
-            layer = _LayerCache(key_states.shape, key_states.dtype, key_states.device)
-            result = (key_states, value_states)
-        else:
-            result = self._dense(layer, key_states, value_states)     # history ++ the new tokens
-        self._ingest(layer, key_states, value_states)
+                result = self._dense(layer, key_states, value_states)     # history ++ the new tokens
+            self._ingest(layer, key_states, value_states)
+        except Exception:
+            # an error before that read (the encoders' arguments, memory): the
+            # positions come first, and their flag is not left to the next call
+            if deferred and bool(self._flags[_POSITION_BAD].item()):
+                self._flags[_POSITION_BAD].zero_()
+                self._position_checked = None
+                raise ValueError(_POSITION_ERROR) from None
+            raise
         self._layers[layer_idx] = layer
         self._after_write(layer_idx, layer)
         return result

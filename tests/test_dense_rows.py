@@ -82,3 +82,17 @@ def test_positions_are_checked_before_a_sealing_update_changes_the_layer(dtype):
     assert cache.get_seq_length() == 60 and cache._layers[0].key_blocks[0] is blocks[0]
     with pytest.raises(ValueError, match="contiguous append"):
         InQuantCache(cache.config).update(k, k, 0, {"cache_position": wrong})
+
+
+def test_positions_come_before_the_errors_of_a_sealing_update():
+    from inquant.cache import CacheConfig, InQuantCache
+    cache = InQuantCache(CacheConfig(block_size=8, residual_length=4, sink_tokens=2, value_bits=2, value_group_size=64))
+    k = torch.randn(1, 2, 20, 96, device="cuda").bfloat16()                     # 96 channels: no whole groups of 64
+    pos = torch.arange(20, device="cuda")
+    with pytest.raises(ValueError, match="contiguous append"):
+        cache.update(k, k, 0, {"cache_position": pos + 1})
+    with pytest.raises(ValueError) as error:
+        cache.update(k, k, 0, {"cache_position": pos})
+    assert "contiguous append" not in str(error.value)
+    cache.update(k[:, :, :5], k[:, :, :5], 0, {"cache_position": pos[:5]})      # no mismatch is left behind
+    assert cache.get_seq_length() == 5
