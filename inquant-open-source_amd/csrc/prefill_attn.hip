@@ -325,9 +325,22 @@ extern "C" int iq_prefill_attention(const void *q, const void *k, const void *v,
     const int64_t obytes = out_dtype == IQ_F32 ? 4 : 2;
     const int vec_out = (uintptr_t)out % (4 * obytes) == 0 && o_st % 4 == 0 && o_sh % 4 == 0;
     const int64_t tiles = (max_seqlen + QT - 1) / QT;
-    // places per group: the least number for which the XCDs' shares are whole
+    // places per group: the least number for which the XCDs' shares are whole;
+    // with several sequences a share is at least 4 items, so the 64 workgroups
+    // resident on an XCD read the K/V of at most 16 of them (eight prompts of
+    // up to 4.1K tokens, 8 heads over 8: 183 us with a contiguous range per
+    // XCD, 210 with shares of one item, 162 with four; seven of 37-4100 tokens,
+    // 32 heads over 8: 291, and 280 with four, 290 with eight).  Where a head's
+    // K/V exceed the XCD's 4 MB L2 (8192 tokens) a sequence's items follow
+    // each other: all its places at once if the heads divide among the XCDs,
+    // else shares of 224 (sixteen prompts of 2K-30K tokens, 28 heads over 4:
+    // 34.5 ms with a contiguous range, 36.5 with shares of 7, 34.4 with 224;
+    // six of up to 12K: 3.07, 3.16 and 3.00)
     int64_t span = 1;
     while (span * Hq % 8) span *= 2;
+    const int64_t least = n_seq == 1 ? 1 : max_seqlen <= 8192 ? 4 : 224;
+    if (least == 224 && Hq % 8 == 0) span = tiles;
+    while (span * Hq / 8 < least && span < tiles) span *= 2;
     const int64_t per_seq = (tiles + span - 1) / span * span * Hq;
     constexpr int64_t MOST = 0xffffffffLL / NT;          // workgroups of a launch (2^32 threads)
     IQ_CHECK_ARG(per_seq <= MOST, "iq_prefill_attention: too many query tiles");

@@ -140,6 +140,22 @@ def test_prefill_varlen_batch_of_4k_tokens_matches_causal_oracle():
     assert worst <= _bound(vn)
 
 
+@pytest.mark.parametrize("hq,h", [(1, 1), (2, 1), (8, 8), (14, 2), (28, 4), (32, 8)])
+@pytest.mark.parametrize("lens", [(1, 8193, 130), (8192, 65), (300, 129, 128)])
+def test_prefill_items_of_a_batch_cover_every_sequence(hq, h, lens):
+    # The order of a batch's items depends on heads, sequences and the longest
+    # length; an item's arithmetic does not, so a batch equals its sequences alone.
+    from inquant_vllm.kernels import prefill_attention
+    q, k, v = _qkv(hq + len(lens), sum(lens), hq, h, torch.bfloat16)
+    offsets = [0, *np.cumsum(lens).tolist()]
+    cu = torch.tensor(offsets, dtype=torch.int32, device="cuda")
+    got = prefill_attention(q, k, v, cu, max(lens), 128 ** -0.5, torch.full_like(q, float("nan")))
+    for a, b in zip(offsets, offsets[1:]):
+        one = torch.tensor([0, b - a], dtype=torch.int32, device="cuda")
+        alone = prefill_attention(q[a:b], k[a:b], v[a:b], one, b - a, 128 ** -0.5, torch.full_like(q[a:b], float("nan")))
+        assert torch.equal(got[a:b], alone)
+
+
 def test_prefill_rejects_bad_arguments():
     from inquant_vllm import prefill_attention
     q, k, v = _qkv(1, 8, 4, 2, torch.bfloat16)
