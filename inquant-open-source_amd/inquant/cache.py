@@ -711,18 +711,25 @@ class InQuantCache(_HFCache):
         value_codec.py:64); a pending position mismatch is reported first."""
         cfg = self.config
         # the encoders only ever raise these words; they are zero here (every
-        # error path below clears what it raised)
+        # error path below clears what was raised)
         flags = self._flag_words(keys.device)
-        if cfg.value_bits is None:
-            new_keys, new_values = _k4_pair_blocks(keys, values, count, cfg.block_size, cfg.codec,
-                                                   flags[_KEY_BAD:_KEY_BAD + 1], flags[_VALUE_BAD:_VALUE_BAD + 1],
-                                                   out)
-            value_error = _BAD_K
-        else:
-            new_keys, new_values = _kv_blocks(keys, values, count, cfg.block_size, cfg.codec, cfg.value_bits,
-                                              cfg.value_group_size, flags[_KEY_BAD:_KEY_BAD + 1],
-                                              flags[_VALUE_BAD:_VALUE_BAD + 1], out)
-            value_error = _BAD_V
+        key_flag, value_flag = flags[_KEY_BAD:_KEY_BAD + 1], flags[_VALUE_BAD:_VALUE_BAD + 1]
+        value_error = _BAD_K if cfg.value_bits is None else _BAD_V
+        try:
+            if cfg.value_bits is None:
+                new_keys, new_values = _k4_pair_blocks(keys, values, count, cfg.block_size, cfg.codec, key_flag,
+                                                       value_flag, out)
+            else:
+                new_keys, new_values = _kv_blocks(keys, values, count, cfg.block_size, cfg.codec, cfg.value_bits,
+                                                  cfg.value_group_size, key_flag, value_flag, out)
+        except Exception:
+            # refused arguments or memory, possibly after the keys' encoder ran
+            bad_position = bool(flags[_POSITION_BAD].item())
+            flags.zero_()
+            if bad_position:
+                self._position_checked = None
+                raise ValueError(_POSITION_ERROR) from None
+            raise
         bad_key, bad_value, bad_position = flags.tolist()
         if bad_key or bad_value or bad_position:
             flags.zero_()

@@ -96,3 +96,20 @@ def test_positions_come_before_the_errors_of_a_sealing_update():
     assert "contiguous append" not in str(error.value)
     cache.update(k[:, :, :5], k[:, :, :5], 0, {"cache_position": pos[:5]})      # no mismatch is left behind
     assert cache.get_seq_length() == 5
+
+
+def test_an_argument_error_between_the_encoders_leaves_no_flag_behind():
+    # the keys' encoder runs (and raises its flag) before the values' arguments are refused
+    from inquant.cache import CacheConfig, InQuantCache
+    cache = InQuantCache(CacheConfig(block_size=8, residual_length=4, sink_tokens=2, value_bits=2, value_group_size=64))
+    k = torch.randn(1, 2, 24, 96, device="cuda").bfloat16()                     # 96 channels: no whole groups of 64
+    k[0, 1, 5, 3] = float("nan")
+    with pytest.raises(ValueError, match="divisible by group_size"):
+        cache.update(k, k, 0)
+    pos = torch.arange(14, device="cuda")
+    cache.update(k[:, :, :13], k[:, :, :13], 0, {"cache_position": pos[:13]})   # 13 tokens: nothing to seal yet
+    with pytest.raises(ValueError, match="divisible by group_size"):
+        cache.append_for_attention(k[:, :, 13:14], k[:, :, 13:14], 0, {"cache_position": pos[13:]})
+    good = torch.randn(1, 2, 24, 64, device="cuda").bfloat16()
+    cache.update(good, good, 1)                                                 # finite data of another layer
+    assert cache.get_seq_length(1) == 24 and not any(cache._flags.tolist())
