@@ -84,6 +84,13 @@ int iq_k4_quantize(const void *x, int x_dtype, const int64_t *x_strides,
                    float *padding, int *bad_flag, void *stream);
 
 /*
+ * Diagnostics: rows of all K4 encodes that have completed on the current device
+ * whose donor pool only the sequential pass over the tokens could decide (the
+ * others' came from order-free sums; the outputs are the same).  Modulo 2^32.
+ */
+int iq_k4_uncertain_rows(uint32_t *rows);
+
+/*
  * Donor selection alone: saliency (and optional donor error) f32 [rows, D]
  * contiguous -> src/don i64 [rows, count].  Replaces reuse_map /
  * _reuse_map (triton_selection.py:46-60, codec.py:137-178).

@@ -19,6 +19,10 @@ namespace {
 
 constexpr int K4_THREADS = 256;
 
+// Rows whose donor pool the order-free sums left uncertain (k4_stats_dev.h), so
+// that they took the sequential pass: iq_k4_uncertain_rows.
+__device__ uint32_t uncertain_rows;
+
 struct K4Args {
     const void *x;
     int dt;
@@ -238,45 +242,86 @@ __device__ __forceinline__ void stats_slice(const void *x, int64_t cb, int64_t s
 
 // The reference's donor error of one channel by its sequential fp64 Welford
 // chain (rows whose pool the order-free sums leave uncertain).  Every lane of
-// the wavefront runs it (lanes past D repeat the last channel).
-template <int DT>
+// the wavefront runs it (lanes past the last channel repeat it), G tokens at a
+// time, the next ones in flight.  While every channel of the wavefront still
+// holds its first value the chain's mean is that value and its sum zero, so it
+// starts where a channel first differs: rows of equal tokens, which are
+// uncertain as a rule (relative to a variance of zero the sums' bound is not
+// small), need no chain.  Eight rows of 32768 tokens x 128 channels, all three
+// launches: equal tokens 1.17 ms, near ties 1.64, certain rows 58 us (bf16; 3.47
+// ms each with the chain in place of the sums).  SHORT: T <= 2^24.
+template <int DT, int G, bool SHORT>
 __device__ __forceinline__ float welford_error(const void *x, int64_t cb, int64_t st, int64_t T, float smean)
 {
     const int lane = threadIdx.x & 63;
-    double mean = 0.0, m2 = 0.0, ygrp = 0.0;
-    auto chain = [&](auto small) {
-        auto f = [&](float v, int64_t t) {
-            // delta / n as RN(1 / n) (off the dependent chain) and one
-            // remainder correction: the correctly rounded quotient
-            // (tests/test_welford_division.py, n up to 2^24)
-            const double n = decltype(small)::value ? (double)(uint32_t)(t + 1) : (double)(t + 1);
-            // rows of up to 2^24 tokens: at the start of each group of
-            // SEQ_PF steps (t a multiple of SEQ_PF there, for_each_seq_t's
-            // groups) lane l computes RN(1 / (t + 1 + l % SEQ_PF)), and
-            // step t reads it from lane t % SEQ_PF: one reciprocal per
-            // group instead of one per step
-            double y;
-            if constexpr (decltype(small)::value) {
-                if ((t & (SEQ_PF - 1)) == 0) ygrp = iq_rcp_small_int((uint32_t)(t + 1 + (lane & (SEQ_PF - 1))));
-                y = iq_read_lane_f64(ygrp, (int)(t & (SEQ_PF - 1)));
-            } else {
-                y = 1.0 / n;
-            }
-            const double dv = (double)v;
-            const double delta = __dsub_rn(dv, mean);
-            const double q0 = __dmul_rn(delta, y);
-            const double r = __builtin_fma(-q0, n, delta);
-            mean = __dadd_rn(mean, __builtin_fma(r, y, q0));
-            const double nd = __dsub_rn(dv, mean);
-            m2 = __dadd_rn(m2, __dmul_rn(delta, nd));
-        };
-        for_each_seq_t<DT>(x, cb, st, T, 1, 0, f);
+    // a global pointer in a called function too (a generic one's loads count as LDS operations as well)
+    typedef typename std::conditional<DT == IQ_F32, float, typename std::conditional<DT == IQ_F64, double, uint16_t>::type>::type E;
+    const auto *xc = (const __attribute__((address_space(1))) E *)(uintptr_t)x + cb;
+    float cur[G], nxt[G];
+    auto load = [&](int64_t t0, float (&v)[G]) {
+        const auto *p = xc + min(t0, T - 1) * st;
+        int64_t left = T - 1 - t0;               // past the last token: the last one again
+#pragma unroll
+        for (int u = 0; u < G; ++u, --left) {
+            const E e = *p;
+            p += left > 0 ? st : 0;
+            if constexpr (DT == IQ_BF16) v[u] = iq_bf16_to_f32(e);
+            else if constexpr (DT == IQ_F16) v[u] = iq_f16_to_f32(e);
+            else v[u] = (float)e;
+        }
     };
-    if (T <= (int64_t(1) << 24)) chain(std::true_type{});
-    else chain(std::false_type{});
+    load(0, cur);
+    const float first = cur[0];
+    double mean = 0.0, m2 = 0.0;
+    auto step = [&](float v, double n, double y) {
+        // delta / n as RN(1 / n) (off the dependent chain) and one remainder
+        // correction: the correctly rounded quotient
+        // (tests/test_welford_division.py, n up to 2^24)
+        const double dv = (double)v;
+        const double delta = __dsub_rn(dv, mean);
+        const double q0 = __dmul_rn(delta, y);
+        const double r = __builtin_fma(-q0, n, delta);
+        mean = __dadd_rn(mean, __builtin_fma(r, y, q0));
+        m2 = __dadd_rn(m2, __dmul_rn(delta, __dsub_rn(dv, mean)));
+    };
+    bool flat = true;
+#pragma unroll 1
+    for (int64_t t0 = 0; t0 < T; t0 += G) {
+        load(t0 + G, nxt);
+        if (flat) {
+            uint32_t diff = 0;
+#pragma unroll
+            for (int u = 0; u < G; ++u) diff |= __float_as_uint(cur[u]) ^ __float_as_uint(first);
+            flat = __ballot(diff != 0) == 0;
+            if (flat || t0 > 0) mean = (double)first;
+        }
+        if (!flat) {
+            // lane l computes the reciprocal of step l % G, and each step reads its own
+            const int64_t mine = t0 + 1 + (lane & (G - 1));
+            const double ys = SHORT || T <= (int64_t(1) << 24) ? iq_rcp_small_int((uint32_t)mine) : 1.0 / (double)mine;
+            const double n0 = (double)t0;
+            if (t0 + G <= T) {
+#pragma unroll
+                for (int u = 0; u < G; ++u) step(cur[u], n0 + (u + 1), iq_read_lane_f64(ys, u));
+            } else {
+#pragma unroll
+                for (int u = 0; u < G - 1; ++u)
+                    if (t0 + u < T) step(cur[u], n0 + (u + 1), iq_read_lane_f64(ys, u));
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < G; ++u) cur[u] = nxt[u];
+    }
     const float var = (float)(m2 / (double)T);
     const float diff = __fsub_rn((float)mean, smean);
     return __fadd_rn(var, __fmul_rn(diff, diff));
+}
+
+// v, the same in every lane, in scalar registers (a called function's arguments are not)
+__device__ __forceinline__ int64_t uniform64(int64_t v)
+{
+    return (int64_t)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+                     (uint32_t)__builtin_amdgcn_readfirstlane((int)v));
 }
 
 // The selection on the sequential errors, for rows whose pool is uncertain.
@@ -287,9 +332,11 @@ __device__ __attribute__((noinline)) void select_sequential(const void *x, int64
                                                             int D, int count, RowLds *s)
 {
     const int tid = threadIdx.x, lane = tid & 63;
+    st = uniform64(st);
+    T = uniform64(T);
     for (int c0 = tid - lane; c0 < D; c0 += ROW_THREADS) {
         const int c = min(c0 + lane, D - 1);
-        const float e = welford_error<DT>(x, base + c * sc, st, T, s->smean[c]);
+        const float e = welford_error<DT, 32, false>(x, base + c * sc, st, T, s->smean[c]);
         if (c0 + lane < D) s->err[c] = e;
     }
     __syncthreads();
@@ -316,6 +363,7 @@ __device__ __forceinline__ void row_select(const K4Args &a, RowLds &s, int64_t r
     }
     __syncthreads();
     if (s.again) {
+        if (tid == 0) atomicAdd(&uncertain_rows, 1u);
         select_sequential<DT, WIDE>(a.x, base, a.sc, a.st, a.T, (int)D, (int)a.count, &s);
         __syncthreads();
     }
@@ -573,7 +621,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k4_encode_kernel(K4Args a)
                 amax = fmaxf(amax, p.amax[lane]);
             }
             s.scale[co] = amax;
-            const IqErrRange r = iq_err_range(s1, s2, amax, s.smean[co], T);
+            const IqErrRange r = iq_err_range(s1, s2, amax, s.smean[co], T, false);
             s.err[co] = r.lo;
             s.ehi[co] = r.hi;
         }
@@ -959,7 +1007,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k4_row_select(K4Args a, RowPlan p
                 amax = fmaxf(amax, q.amax[lane]);
             }
             s.scale[co] = amax;
-            const IqErrRange r = iq_err_range(s1, s2, amax, s.smean[co], a.T);
+            const IqErrRange r = iq_err_range(s1, s2, amax, s.smean[co], a.T, false);
             s.err[co] = r.lo;
             s.ehi[co] = r.hi;
             if (!iq_isfinite(amax) || s2 != s2) s.bad = 1;
@@ -1320,8 +1368,8 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
         s_amax[c1] = amax;
         if (amax_bits >= (F16IN ? 0x7c00u : 0x7f80u)) s_bad = 1;     // an inf or NaN in the channel
         if (a.min_error) {
-            const IqErrRange r =
-                iq_err_range(__dadd_rn(sum1, s_sum1[c1]), __dadd_rn(sum2, s_sum2[c1]), amax, s_smean[c1], T);
+            const double s1 = __dadd_rn(sum1, s_sum1[c1]), s2 = __dadd_rn(sum2, s_sum2[c1]);
+            const IqErrRange r = iq_err_range(s1, s2, amax, s_smean[c1], T, iq_same16(s1, s2, amax, T));
             s_err[c1] = r.lo;
             s_ehi[c1] = r.hi;
         }
@@ -1360,19 +1408,13 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
     __builtin_amdgcn_s_setprio(1);
     __syncthreads();
     if (__builtin_expect(s_again, 0)) {
-        // the pool is uncertain: the reference's sequential errors, and the selection on them
-        if (tid < TILE_D) {
-            double mean = 0.0, m2 = 0.0;
-#pragma unroll 1
-            for (int t = 0; t < T; ++t) {
-                const double dv = (double)tile_f32<F16IN>(xr[(int64_t)t * a.st + tid]);
-                const double delta = __dsub_rn(dv, mean);
-                mean = __dadd_rn(mean, delta / (double)(t + 1));
-                m2 = __dadd_rn(m2, __dmul_rn(delta, __dsub_rn(dv, mean)));
-            }
-            const float diff = __fsub_rn((float)mean, s_smean[tid]);
-            s_err[tid] = __fadd_rn((float)(m2 / (double)T), __fmul_rn(diff, diff));
-        }
+        // the pool is uncertain (errors that tie in real arithmetic and differ in their roundings; channels of one
+        // value are exact, iq_same16): the reference's sequential errors, and the selection on them.  1024 rows of 256
+        // bf16 tokens: 60 us where all take it, 37 where none does and 32 where all tokens are equal; with the chain in
+        // place of the sums 38, 43 and 36
+        if (tid == 0) atomicAdd(&uncertain_rows, 1u);
+        if (tid < TILE_D)
+            s_err[tid] = welford_error<F16IN ? IQ_F16 : IQ_BF16, 16, true>(xr, tid, a.st, T, s_smean[tid]);
         __syncthreads();
         if (tid < 64) iq_select_wave128(s_sal, s_err, (int)a.count, s_src, s_don, s_is_src, s_src_of, s_list);
         __syncthreads();
@@ -1762,6 +1804,14 @@ int launch_rows(const K4Args &a, int64_t B, hipStream_t st)
 }
 
 }  // namespace
+
+extern "C" int iq_k4_uncertain_rows(uint32_t *rows)
+{
+    IQ_CHECK_ARG(rows, "iq_k4_uncertain_rows: null pointer");
+    const hipError_t e = hipMemcpyFromSymbol(rows, HIP_SYMBOL(uncertain_rows), sizeof *rows);
+    if (e != hipSuccess) return iq_fail(IQ_ERR_DEVICE, "iq_k4_uncertain_rows: %s", hipGetErrorString(e));
+    return IQ_OK;
+}
 
 extern "C" int iq_k4_quantize(const void *x, int x_dtype, const int64_t *x_strides, int64_t B, int64_t H,
                               int64_t T, int64_t D, int64_t count, int64_t sample_stride, int min_error,

@@ -25,7 +25,11 @@
 //          8 (n + 8) u A^2 after the division by n.  S2 / n - (S1 / n)^2 is
 //          off by at most 4 (n + 16) u A^2.  H = 16 (n + 16) u A^2 encloses
 //          both with a quarter to spare.
-// A channel of zeros has E = H = 0: its error is exactly zero.
+// A channel of zeros has E = H = 0: its error is exactly zero.  So is the error
+// of a channel whose tokens all hold one value v (`same`): the chain's mean is v
+// from its first step on, its sum stays zero, and err = fl(fl(v - smean)^2).
+// Without that a block of equal tokens (padding, a run of one token) left every
+// pool uncertain: relative to a variance of zero the bound is not small.
 #pragma once
 
 #include "iq_common.h"
@@ -34,8 +38,23 @@ struct IqErrRange {
     float lo, hi;
 };
 
-__device__ __forceinline__ IqErrRange iq_err_range(double s1, double s2, float amax, float smean, int64_t n)
+// Whether all of n <= 256 values of a 16-bit type are equal, from their sums.
+// A value other than the largest in magnitude differs from it by at least
+// 2^-11 A, so a channel that is not constant has a variance of at least
+// 2^-22 A^2 / (2 n) >= 2^-31 A^2; the computed one is within
+// 4 (n + 16) u A^2 < 2^-42 A^2 of the true one, and H < 2^-40 A^2.
+__device__ __forceinline__ bool iq_same16(double s1, double s2, float amax, int64_t n)
 {
+    const double inv = 1.0 / (double)n, A = (double)amax, mean = s1 * inv;
+    return __builtin_fma(-mean, mean, s2 * inv) <= A * A * ((double)(n + 16) * 0x1p-49);
+}
+
+__device__ __forceinline__ IqErrRange iq_err_range(double s1, double s2, float amax, float smean, int64_t n, bool same)
+{
+    if (same) {
+        const float d = __fsub_rn(copysignf(amax, (float)s1), smean), q = __fmul_rn(d, d);
+        return IqErrRange{q, q};
+    }
     const double inv = 1.0 / (double)n, A = (double)amax;
     const double mean = s1 * inv;
     const double var = __builtin_fma(-mean, mean, s2 * inv);

@@ -56,6 +56,7 @@ _SIGNATURES = {
     "iq_last_error": (ctypes.c_char_p, []),
     "iq_k4_quantize": (_int, [_p, _int, ctypes.POINTER(_i64), _i64, _i64, _i64, _i64, _i64, _i64, _int,
                               _p, _p, _p, _p, _int, _p, _p, _p]),
+    "iq_k4_uncertain_rows": (_int, [ctypes.POINTER(ctypes.c_uint32)]),
     "iq_reuse_map": (_int, [_p, _p, _i64, _i64, _i64, _p, _p, _p]),
     "iq_k4_dequantize": (_int, [_p, _p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _p, _int, _p]),
     "iq_k4_dequantize_into": (_int, [_p, _p, _p, _p, _int, _p, _i64, _i64, _i64, _i64, _i64, _p, _int, _i64, _i64,

@@ -146,3 +146,69 @@ def test_blocks_with_tied_errors(T, dtype):
         f = xt.float().cpu().numpy()
         want = oracle.pack_pages(oracle.k4_quantize(f, 8, 0.125, "min_error"), oracle.v_quantize(f, 2, 64), 3, T)
         np.testing.assert_array_equal(pack_pages(xt, xt, PageLayout(T, 3)).cpu().numpy(), want)
+
+
+def _uncertain(encode):
+    """Rows of encode() that took the sequential pass."""
+    import ctypes
+    from inquant import _native
+
+    def count():
+        torch.cuda.synchronize()
+        rows = ctypes.c_uint32()
+        _native.check(_native.lib().iq_k4_uncertain_rows(ctypes.byref(rows)))
+        return rows.value
+    before = count()
+    encode()
+    return (count() - before) % 2 ** 32
+
+
+# one row a workgroup (16-byte pieces and bytes), rows spread over the chip, the tile encoder whole and ragged
+ROUTES = [(64, 200, torch.float32), (66, 40, torch.bfloat16), (272, 100, torch.float16), (40, 64, torch.float64),
+          (128, 700, torch.bfloat16), (66, 3000, torch.float32), (64, 2000, torch.float64), (512, 600, torch.float16),
+          (128, 256, torch.bfloat16), (128, 256, torch.float16), (128, 100, torch.bfloat16), (128, 1, torch.float16)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,T,dtype", ROUTES)
+def test_rows_of_repeated_tokens(D, T, dtype):
+    # padding, warm-up batches, runs of one token: every channel is constant.  The tile encoder's errors are exact there;
+    # the general rows find no channel that differs and run no chain
+    token = synth.normal(D + T, (2, 3, 1, D))
+    token[0, 0] = np.round(token[0, 0])                 # many channels tie; zeros of both signs
+    token[0, 1] *= 1e-38
+    token[1, 2] *= 1e4
+    x = torch.from_numpy(np.repeat(token, T, 2)).cuda().to(dtype)
+    varied = torch.from_numpy(synth.normal(D * T, (2, 3, T, D))).cuda().to(dtype)
+    half = varied.clone()
+    half[:, :, :, D // 2:] = x[:, :, :, D // 2:]        # half of the channels constant
+    assert _uncertain(lambda: _check(varied, 8, 0.125, "min_error")) == 0
+    tile = D == 128 and T <= 256
+    for y, stride in ((x, 8), (half, 3)):
+        rows = _uncertain(lambda: _check(y, stride, 0.25, "min_error"))
+        assert rows == 0 or not tile
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,T,dtype", [r for r in ROUTES if r[1] > 1])
+def test_near_ties_take_the_sequential_pass(D, T, dtype):
+    # ones, but for one unsampled token a channel (row 1: in the last tokens): errors that are equal in real arithmetic
+    # and not within the sums' bounds
+    x = np.ones((1, 2, T, D))
+    for c in range(D):
+        x[0, 0, 1 + 8 * (c % ((T - 1) // 8)), c] += 2.0 ** -7
+        x[0, 1, T - 1 - 8 * ((7 * c) % max(T // 32, 1)) - (T % 8 == 1), c] -= 2.0 ** -7
+    assert _uncertain(lambda: _check(torch.from_numpy(x).cuda().to(dtype), 8, 0.125, "min_error")) == 2
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", [64, 256])
+def test_pages_of_repeated_tokens_need_no_sequential_pass(block):
+    from inquant_vllm.layout import PageLayout, pack_pages
+    x = np.repeat(np.round(2 * synth.normal(block, (3, 2, 1, 128))) / 2, block, 2)
+    xt = torch.from_numpy(x).cuda().to(torch.bfloat16)
+    f = xt.float().cpu().numpy()
+    want = oracle.pack_pages(oracle.k4_quantize(f, 8, 0.125, "min_error"), oracle.v_quantize(f, 2, 64), 2, block)
+    got = []
+    assert _uncertain(lambda: got.append(pack_pages(xt, xt, PageLayout(block, 2)))) == 0
+    np.testing.assert_array_equal(got[0].cpu().numpy(), want)
