@@ -300,7 +300,7 @@ class PackedDecodeState:
         stream = self._pin.check(fmt.device)
         new_keys, new_values = tuple(key_blocks[have:]), tuple(value_blocks[have:])
         fmt.admit(new_keys, new_values)
-        if self._desc is None or self._desc.tables.device != fmt.device:
+        if not have:      # also after dense-only steps, whose tables are of no format
             self._desc = _Descriptors(fmt.device, fmt.heads, fmt.value_bits == 0)
         self._format = fmt
         self._desc.reserve(have, len(key_blocks))

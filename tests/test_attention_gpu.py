@@ -352,3 +352,18 @@ def test_extend_checks_every_appended_block_and_keeps_the_state_on_error():
         assert torch.equal(state.decode(q), ref)
     state.extend(keys, values)
     assert torch.equal(state.decode(q), PackedDecodeState(keys, values).decode(q))
+
+
+@pytest.mark.parametrize("value_bits", [0, 2, 4])
+def test_state_decoded_before_its_first_block(value_bits):
+    # a short prompt: dense steps first, then the blocks that are sealed on the way
+    from inquant.triton_attention import PackedDecodeState
+    case = make_case(77, n_blocks=2, block=64, value_bits=value_bits)
+    state = PackedDecodeState([], [])
+    np.testing.assert_allclose(_decode_f32(state, case), oracle_decode(case.query, [], [], *case.kwargs().values()),
+                               atol=ATOL, rtol=0)
+    for n in (1, 2):
+        state.extend(case.key_blocks[:n], case.value_blocks[:n])
+        whole = PackedDecodeState(case.key_blocks[:n], case.value_blocks[:n])
+        np.testing.assert_array_equal(_decode_f32(state, case), _decode_f32(whole, case))
+        assert torch.equal(state._tables[:n], whole._tables) and state._value_map.shape[1:] == whole._value_map.shape[1:]
