@@ -51,7 +51,7 @@ except ImportError:  # the codec and cache do not need transformers
         pass
 
 from . import _native as nat
-from .codec import _BAD_K, CodecConfig, PackedTensor, _per_block, quantize
+from .codec import _BAD_K, CodecConfig, PackedTensor, _blocks_of, _per_block, quantize
 from .value_codec import _BAD_V, PackedValues, quantize_values
 
 _POSITION_ERROR = "Only contiguous append positions are supported; reset before a new request"
@@ -208,13 +208,12 @@ class _LayerCache:
         return self.runs[-1][1] if self.runs else 0
 
     def _expand(self) -> None:
-        """Block objects of the batches that have none yet: a prefill's blocks
-        are 16 views and two objects each (0.6 ms for 127 of them), which only
-        a reader of single blocks needs."""
+        """Block objects of the batches that have none yet: only a reader of
+        single blocks and the packed view need them."""
         for (first, stop), (keys, values) in zip(self.runs, self.batches):
             if first == len(self._keys):
-                self._keys.extend(_unbatched(keys, stop - first))
-                self._values.extend(_unbatched(values, stop - first))
+                self._keys.extend(_blocks_of(keys, stop - first))
+                self._values.extend(_blocks_of(values, stop - first))
 
     @property
     def key_blocks(self) -> list:
@@ -310,16 +309,6 @@ def _carve(device, fields):
     raw = torch.empty(total, dtype=torch.uint8, device=device)
     typed = [raw.view(dtype) for dtype in dtypes]   # one reinterpretation per dtype
     return [torch.as_strided(typed[i], shape, strides, offset) for i, shape, strides, offset in views]
-
-
-def _unbatched(batch, count: int) -> list:
-    """The blocks of a batched [count, H, T, D] encode, views of its fields."""
-    if count == 1:
-        return [batch]
-    shape = (1, *batch.shape[1:])
-    if isinstance(batch, PackedValues):
-        return _per_block(batch, count, shape, PackedValues, bits=batch.bits, group_size=batch.group_size)
-    return _per_block(batch, count, shape, PackedTensor)
 
 
 def _dequantize_into(run, dense, at: int) -> None:

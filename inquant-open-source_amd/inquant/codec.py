@@ -69,8 +69,63 @@ def _per_block(packed, count: int, shape, cls, **extra) -> list:
             for parts in zip(*pieces)]
 
 
+def _blocks_of(batch, count: int) -> list:
+    """The blocks of a batched [count, H, T, D] encode.  Their fields become
+    views of the batch's when they are read (_BlockFields)."""
+    if count == 1:
+        return [batch]
+    blocks = []
+    for i in range(count):
+        block = object.__new__(type(batch))
+        block.__dict__.update(_batch=batch, _index=i)
+        blocks.append(block)
+    return blocks
+
+
+def _batch_runs(blocks):
+    """(first block, packed, index, count) of each run of ``blocks`` that are
+    consecutive in one batched encode; another block is its own ``packed``."""
+    start, n = 0, len(blocks)
+    while start < n:
+        block, stop = blocks[start], start + 1
+        batch = getattr(block, "_batch", None)
+        if batch is None:
+            yield block, block, 0, 1
+        else:
+            index = block._index
+            while (stop < n and getattr(blocks[stop], "_batch", None) is batch
+                   and blocks[stop]._index == index + stop - start):
+                stop += 1
+            yield block, batch, index, stop - start
+        start = stop
+
+
+class _BlockFields:
+    """Base of the packed dataclasses.  A block of a batched encode
+    (_blocks_of) holds the batch and its index there: making the views of all
+    blocks of a long prefill takes longer than encoding them, and the decode
+    state needs only their addresses."""
+
+    _batch = None
+
+    def __getattr__(self, name):        # a field that this instance has not got yet
+        batch = self._batch
+        if batch is None or name not in self.__dataclass_fields__:
+            raise AttributeError(f"{type(self).__name__!r} object has no attribute {name!r}")
+        value = getattr(batch, name)
+        if name == "shape":
+            value = (1, *value[1:])
+        elif isinstance(value, torch.Tensor):
+            value = value.narrow(0, self._index, 1)
+        self.__dict__[name] = value
+        return value
+
+    def __getstate__(self) -> dict:     # copies and pickles hold the fields alone
+        return {name: getattr(self, name) for name in self.__dataclass_fields__}
+
+
 @dataclass(frozen=True)
-class PackedTensor:
+class PackedTensor(_BlockFields):
     """One packed K4 tensor; layout of codec.py:58-110.
 
     payload u8 [B, H, T, D/2] (even channel in the low nibble), scales f32

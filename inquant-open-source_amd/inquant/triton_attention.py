@@ -29,11 +29,12 @@ from __future__ import annotations
 
 import math
 import operator
+from array import array
 
 import torch
 
 from . import _native as nat
-from .codec import PackedTensor
+from .codec import PackedTensor, _batch_runs
 from .value_codec import PackedValues
 
 _SPLIT = 32           # tokens per dense partition (the native kernels' split)
@@ -93,13 +94,14 @@ class _BlockFormat:
     __slots__ = ("device", "heads", "tokens", "salient", "desc_bytes", "value_bits", "value_group")
 
     def __init__(self, key0, value0):
-        if key0.shape[0] != 1 or key0.shape[-1] != 128 or key0.payload.device.type != "cuda":
+        shape, packed = key0.shape, getattr(key0, "_batch", None) or key0
+        if shape[0] != 1 or shape[-1] != 128 or packed.payload.device.type != "cuda":
             raise ValueError("Packed decode requires CUDA blocks with batch=1 and head_dim=128")
-        self.device = key0.payload.device
-        self.heads = key0.shape[1]
-        self.tokens = key0.shape[2]
-        self.salient = key0.salient_channels.shape[-1]
-        self.desc_bytes = key0.salient_channels.element_size()
+        self.device = packed.payload.device
+        self.heads = shape[1]
+        self.tokens = shape[2]
+        self.salient = packed.salient_channels.shape[-1]
+        self.desc_bytes = packed.salient_channels.element_size()
         coded = isinstance(value0, PackedValues)
         self.value_bits = value0.bits if coded else 0
         self.value_group = value0.group_size if coded else 64
@@ -108,13 +110,14 @@ class _BlockFormat:
         return all(getattr(self, f) == getattr(other, f) for f in self.__slots__)
 
     def admit(self, keys, values) -> None:
-        """Raise the reference's errors for blocks that break the layout."""
-        for k in keys:
-            if (not isinstance(k, PackedTensor) or k.shape != (1, self.heads, self.tokens, 128)
+        """Raise the reference's errors for blocks (runs of them, _batch_runs)
+        that break the layout."""
+        for block, k, _, _ in keys:
+            if (not isinstance(k, PackedTensor) or block.shape != (1, self.heads, self.tokens, 128)
                     or k.salient_channels.shape[-1] != self.salient):
                 raise ValueError("All packed K/V blocks must share shape and salient-channel count")
-        for v in values:
-            if v.shape != (1, self.heads, self.tokens, 128):
+        for block, v, _, _ in values:
+            if block.shape != (1, self.heads, self.tokens, 128):
                 raise ValueError("All packed blocks must share shape")
             if self.value_bits:
                 if not isinstance(v, PackedValues) or v.bits != self.value_bits or v.group_size != self.value_group:
@@ -122,19 +125,38 @@ class _BlockFormat:
             elif not isinstance(v, PackedTensor) or v.salient_channels.shape[-1] != self.salient:
                 raise ValueError("All InQuant V blocks must share the salient-channel count")
         index = self.device.index
-        for block in (*keys, *values):
-            for t in block.tensors.values():
+        for _, packed, _, _ in (*keys, *values):
+            for t in packed.tensors.values():
                 if t.get_device() != index:
                     raise ValueError("All packed tensors must share the same CUDA device")
         if self.salient > 64:
             raise ValueError("Packed decode supports at most 64 salient channels (int8 roles)")
 
 
-def _field_addresses(k, v, k4_values):
-    """A block's addresses in pointer-table column order."""
-    return (k.payload.data_ptr(), k.scales.data_ptr(), k.padding.data_ptr(), v.payload.data_ptr(),
-            v.scales.data_ptr(), (v.padding if k4_values else v.offsets).data_ptr(),
-            k.salient_channels.data_ptr(), k.donor_channels.data_ptr())
+_KEY_FIELDS = ("payload", "scales", "padding", "salient_channels", "donor_channels")
+
+
+def _column(runs, name: str) -> list:
+    """The addresses of a field over runs of blocks."""
+    out = []
+    for _, packed, first, count in runs:
+        t = getattr(packed, name)
+        base, step = t.data_ptr(), t.stride(0) * t.element_size()
+        if count == 1 or t.numel() == 0:
+            out.extend([base + first * step if base else 0] * count)
+        else:
+            out.extend(range(base + first * step, base + (first + count) * step, step))
+    return out
+
+
+def _block_columns(keys, values, k4_values: bool) -> list:
+    """The fields' addresses, in the order of iq_block_ptrs (the first eight
+    are the pointer table's columns)."""
+    k = [_column(keys, name) for name in _KEY_FIELDS]
+    none = [0] * len(k[0])
+    v = [_column(values, name) for name in ("payload", "scales", "padding" if k4_values else "offsets")]
+    v_roles = [_column(values, name) for name in _KEY_FIELDS[3:]] if k4_values else [none, none]
+    return [*k[:3], *v, *k[3:], *v_roles]
 
 
 def _field_bytes(fmt: "_BlockFormat") -> tuple:
@@ -175,39 +197,34 @@ class _Descriptors:
         if self.k4_values:
             self.value_map = regrow(self.value_map, (grown, *self.value_map.shape[1:]))
 
-    def grow_run(self, first: int, keys, values, fmt: _BlockFormat) -> None:
+    def grow_run(self, first: int, columns, fmt: _BlockFormat) -> None:
         """Extend the fixed-stride run over the new blocks while they continue it."""
         if not self.run_open or fmt.value_bits == 0:
             self.run_open = False
             return
-        step = _field_bytes(fmt)
-        run = self.run
-        for i, (k, v) in enumerate(zip(keys, values)):
-            addr = _field_addresses(k, v, False)
-            if run.blocks == 0 and first + i == 0:
-                for f in range(_COLUMNS):
-                    run.base[f] = addr[f]
-            elif run.blocks != first + i or any(addr[f] != run.base[f] + run.blocks * step[f]
-                                                for f in range(_COLUMNS)):
-                self.run_open = False
-                return
-            run.blocks += 1
+        run, count = self.run, len(columns[0])
+        if run.blocks == 0 and first == 0:
+            run.base[:] = [c[0] for c in columns[:_COLUMNS]]
+        more = count if run.blocks == first else 0
+        for base, step, column in zip(run.base, _field_bytes(fmt), columns):
+            at = base + first * step
+            wanted = list(range(at, at + count * step, step)) if step else [at] * count
+            if column[:more] != wanted[:more]:
+                more = next(i for i in range(more) if column[i] != wanted[i])
+        run.blocks += more
+        self.run_open = more == count
 
     def write(self, first: int, keys, values, fmt: _BlockFormat, stream: int) -> None:
-        self.grow_run(first, keys, values, fmt)
-        rows = (nat.BlockPtrs * len(keys))()
-        for row, k, v in zip(rows, keys, values):
-            row.k_payload, row.k_scales, row.k_padding = k.payload.data_ptr(), k.scales.data_ptr(), k.padding.data_ptr()
-            row.k_src, row.k_don = k.salient_channels.data_ptr(), k.donor_channels.data_ptr()
-            row.v_payload, row.v_scales = v.payload.data_ptr(), v.scales.data_ptr()
-            if self.k4_values:
-                row.v_offsets = v.padding.data_ptr()
-                row.v_src, row.v_don = v.salient_channels.data_ptr(), v.donor_channels.data_ptr()
-            else:
-                row.v_offsets = v.offsets.data_ptr()
+        columns = _block_columns(keys, values, self.k4_values)
+        self.grow_run(first, columns, fmt)
+        count = len(columns[0])
+        rows = (nat.BlockPtrs * count)()
+        words = memoryview(rows).cast("B").cast("Q")
+        for f, column in enumerate(columns):
+            words[f::len(columns)] = array("Q", column)
         nat.check(nat.lib().iq_decode_append(
             self.tables.data_ptr(), self.key_map.data_ptr(),
-            self.value_map.data_ptr() if self.k4_values else None, first, len(keys), rows, fmt.heads,
+            self.value_map.data_ptr() if self.k4_values else None, first, count, rows, fmt.heads,
             fmt.salient, fmt.desc_bytes, stream))
 
     def tensors(self):
@@ -299,12 +316,13 @@ class PackedDecodeState:
                 raise ValueError("All packed K/V blocks must share shape and salient-channel count")
         stream = self._pin.check(fmt.device)
         new_keys, new_values = tuple(key_blocks[have:]), tuple(value_blocks[have:])
-        fmt.admit(new_keys, new_values)
+        key_runs, value_runs = list(_batch_runs(new_keys)), list(_batch_runs(new_values))
+        fmt.admit(key_runs, value_runs)
         if not have:      # also after dense-only steps, whose tables are of no format
             self._desc = _Descriptors(fmt.device, fmt.heads, fmt.value_bits == 0)
         self._format = fmt
         self._desc.reserve(have, len(key_blocks))
-        self._desc.write(have, new_keys, new_values, fmt, stream)
+        self._desc.write(have, key_runs, value_runs, fmt, stream)
         # only the new blocks are added (the held prefix is identical): no
         # pass over the whole history beyond the identity check
         self._keys.extend(new_keys)

@@ -12,11 +12,11 @@ from dataclasses import dataclass
 import torch
 
 from . import _native as nat
-from .codec import _per_block, _view_nbytes
+from .codec import _BlockFields, _per_block, _view_nbytes
 
 
 @dataclass(frozen=True)
-class PackedValues:
+class PackedValues(_BlockFields):
     payload: torch.Tensor
     scales: torch.Tensor
     offsets: torch.Tensor
