@@ -110,8 +110,8 @@ class PackedAttentionView(NamedTuple):
 
 def _launches(tensor: torch.Tensor) -> bool:
     """Whether a launch on the tensor's stream runs on its GPU: the default
-    stream's handle names the current device's, so tensors of another one (a
-    model spread over GPUs) are left to torch, which switches devices."""
+    stream's handle names the current device's.  The cache's calls make the
+    GPU of their tensors (a model spread over GPUs) the current one."""
     return tensor.is_cuda and tensor.device.index == torch.cuda.current_device()
 
 
@@ -551,6 +551,12 @@ class InQuantCache(_HFCache):
     def update(self, key_states, value_states, layer_idx, cache_kwargs=None, *args, **kwargs):
         """Store new tokens; return the layer's full K/V (the inputs themselves
         on the first call, else dequantized history ++ the new tokens)."""
+        if not key_states.is_cuda or _launches(key_states):
+            return self._update(key_states, value_states, layer_idx, cache_kwargs)
+        with torch.cuda.device(key_states.device):
+            return self._update(key_states, value_states, layer_idx, cache_kwargs)
+
+    def _update(self, key_states, value_states, layer_idx, cache_kwargs):
         layer, position = self._check(key_states, value_states, layer_idx, cache_kwargs)
         start = 0 if layer is None else layer.seq_length
         deferred = (position is not None and position.device == key_states.device and _launches(position)
@@ -583,6 +589,12 @@ class InQuantCache(_HFCache):
 
         Blocks sealed by this append are attended from the next step on
         (cache.py:242-269)."""
+        if not key_states.is_cuda or _launches(key_states):
+            return self._append(key_states, value_states, layer_idx, cache_kwargs)
+        with torch.cuda.device(key_states.device):
+            return self._append(key_states, value_states, layer_idx, cache_kwargs)
+
+    def _append(self, key_states, value_states, layer_idx, cache_kwargs) -> PackedAttentionView:
         layer, position = self._check(key_states, value_states, layer_idx, cache_kwargs)
         if layer is None or key_states.shape[2] != 1:
             raise ValueError("append_for_attention requires one new token after an existing prefill")
@@ -815,7 +827,10 @@ class InQuantCache(_HFCache):
         layer = self._layers.get(layer_idx)
         if layer is None:
             raise KeyError(f"No cached layer {layer_idx}")
-        return self._dense(layer)
+        if layer.device.type != "cuda" or layer.device.index == torch.cuda.current_device():
+            return self._dense(layer)
+        with torch.cuda.device(layer.device):
+            return self._dense(layer)
 
     def _dense(self, layer, new_keys=None, new_values=None):
         """sink ++ dequantized blocks ++ tail (++ new_keys / new_values, tokens

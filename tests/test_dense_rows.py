@@ -63,6 +63,53 @@ def test_rows_and_positions_of_another_device_are_left_to_torch(monkeypatch):
         assert torch.equal(got, k)
 
 
+@pytest.mark.parametrize("vbits", [2, None])
+def test_every_launch_of_the_cache_runs_on_the_gpu_of_its_tensors(monkeypatch, vbits):
+    # GPU 1 is said to be the current one: updates, appends, seals and materialize switch to GPU 0 for their launches
+    from inquant import _native
+    from inquant.cache import CacheConfig, InQuantCache
+    k = torch.randn(1, 2, 60, 128, device="cuda").bfloat16()
+    pos = torch.arange(60, device="cuda")
+
+    def session():
+        cache = InQuantCache(CacheConfig(block_size=8, residual_length=4, sink_tokens=2, value_bits=vbits))
+        out = [*cache.update(k[:, :, :30], k[:, :, :30], 0, {"cache_position": pos[:30]})]
+        out += cache.update(k[:, :, 30:45], k[:, :, 30:45], 0, {"cache_position": pos[30:45]})
+        for i in range(45, 60):
+            view = cache.append_for_attention(k[:, :, i:i + 1], k[:, :, i:i + 1], 0, {"cache_position": pos[i:i + 1]})
+            out += [view.residual_key.clone(), view.residual_value.clone()]
+        return out + [*cache.materialize(0)]
+
+    want = session()
+    current, launches, lib = [1], [], _native.lib()
+
+    class Switch:
+        def __init__(self, device):
+            self.index = torch.device(device).index
+
+        def __enter__(self):
+            self.before, current[0] = current[0], self.index
+
+        def __exit__(self, *error):
+            current[0] = self.before
+
+    class Spy:
+        def __getattr__(self, name):
+            launches.append((name, current[0]))
+            return getattr(lib, name)
+
+    row = _native.tail_append_row
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    monkeypatch.setattr(torch.cuda, "device", Switch)
+    monkeypatch.setattr(_native, "lib", Spy)
+    monkeypatch.setattr(_native, "tail_append_row", lambda *args: (launches.append(("append", current[0])), row(*args))[1])
+    got = session()
+    monkeypatch.undo()
+    assert {name for name, _ in launches} >= {"append", "iq_copy_rows", "iq_check_positions", "iq_k4_dequantize_into"}
+    assert all(device == 0 for _, device in launches) and current == [1]
+    assert all(torch.equal(a, b) for a, b in zip(got, want, strict=True))
+
+
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
 def test_positions_are_checked_before_a_sealing_update_changes_the_layer(dtype):
     from inquant.cache import CacheConfig, InQuantCache
