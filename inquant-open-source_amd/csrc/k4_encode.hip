@@ -19,7 +19,7 @@ namespace {
 
 constexpr int K4_THREADS = 256;
 
-// Rows whose donor pool the order-free sums left uncertain (k4_stats_dev.h), so
+// Rows whose donor pool the order-free sums left uncertain (k4_stats.h), so
 // that they took the sequential pass: iq_k4_uncertain_rows.
 __device__ uint32_t uncertain_rows;
 
@@ -183,7 +183,7 @@ __device__ __forceinline__ float tile_f32(uint32_t bits16)
 // to LONG_ROW tokens is one workgroup's (k4_encode_kernel); a longer one is
 // spread over the chip in three launches (k4_row_stats, k4_row_select,
 // k4_quantize_rows).  Both take the donor errors from order-free sums with a
-// certificate (k4_stats_dev.h), so nothing but the saliency sums has an order
+// certificate (k4_stats.h), so nothing but the saliency sums has an order
 // to keep, and torch's cascade leaves those in independent pieces.  Eight rows
 // of 32768 bf16 tokens x 128 channels: 22.7 + 16.4 + 21.8 us (3.0, then 3.8
 // TB/s of rows read and words written; 3390 + 89 us with a sequential fp64
@@ -1059,7 +1059,7 @@ __global__ __launch_bounds__(K4_THREADS) void k4_quantize_rows(K4Args a, int64_t
 //           fp64 (min_error only) and takes amax and finiteness as an integer
 //           max of the 16-bit magnitudes; one half also adds the sampled
 //           sums (torch cascade order).  The donor errors come from the sums
-//           with a certificate (k4_stats_dev.h);
+//           with a certificate (k4_stats.h);
 //   then    donor selection by the whole workgroup (iq_select_tile128);
 //           the sequential donor picks run on one wavefront alone, and with a
 //           value row to encode (page mode, or VB = 2 / 4) the other three

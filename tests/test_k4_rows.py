@@ -1,6 +1,12 @@
 """General-row K4 encoder: rows of one workgroup, rows spread over the chip,
 and the certified donor errors both take from order-free sums
-(csrc/k4_stats_dev.h)."""
+(csrc/k4_stats.h, whose arithmetic is compiled for the host here)."""
+import ctypes
+import functools
+import os
+import subprocess
+import tempfile
+
 import numpy as np
 import pytest
 import torch
@@ -10,22 +16,61 @@ import synth
 
 F = np.float32
 
+# The sums of a channel's tokens as the encoders take them (`parts` interleaved partial sums, added in order) and the
+# header's enclosure; `few`: with the constant channels told from the sums, as in the tile encoder.
+SRC = r"""
+#include "k4_stats.h"
+#include <math.h>
+extern "C" void ranges(const float *x, const float *smean, int64_t n, int64_t channels, int parts, int few, float *lo,
+                       float *hi, uint64_t *lo_key, uint64_t *hi_key, uint8_t *same)
+{
+    for (int64_t c = 0; c < channels; ++c) {
+        double s1 = 0.0, s2 = 0.0;
+        float amax = 0.0f;
+        for (int p = 0; p < parts; ++p) {
+            double a = 0.0, b = 0.0;
+            for (int64_t t = p; t < n; t += parts) {
+                const double v = x[t * channels + c];
+                a += v;
+                b = fma(v, v, b);
+                amax = fmaxf(amax, fabsf(x[t * channels + c]));
+            }
+            s1 += a;
+            s2 += b;
+        }
+        same[c] = few && iq_same16(s1, s2, amax, n);
+        const IqErrRange r = iq_err_range(s1, s2, amax, smean[c], n, same[c]);
+        lo[c] = r.lo;
+        hi[c] = r.hi;
+        lo_key[c] = iq_err_key(r.lo, (int)c);
+        hi_key[c] = iq_err_key(r.hi, (int)c);
+    }
+}
+"""
 
-def _err_range(x, smean):
-    """iq_err_range of the rows x [n, channels] (float32)."""
-    n = x.shape[0]
-    d = x.astype(np.float64)
-    s1, s2 = d.sum(0), (d * d).sum(0)
-    a = np.abs(x).max(0).astype(np.float64)
-    inv = 1.0 / n
-    mean = s1 * inv
-    var = s2 * inv - mean * mean
-    e, h = a * ((2 * n + 32) * 2.0 ** -53), a * a * ((n + 16) * 2.0 ** -49)
-    with np.errstate(over="ignore", invalid="ignore"):
-        vlo, vhi = np.maximum(var - h, 0).astype(F), np.maximum(var + h, 0).astype(F)
-        da, db = (mean - e).astype(F) - smean, (mean + e).astype(F) - smean
-        qa, qb = da * da, db * db
-        return vlo + np.where((da < 0) & (db > 0), F(0), np.minimum(qa, qb)), vhi + np.maximum(qa, qb)
+
+@functools.lru_cache(None)
+def _host():
+    with tempfile.TemporaryDirectory() as tmp:
+        src, out = os.path.join(tmp, "ranges.cpp"), os.path.join(tmp, "ranges.so")
+        with open(src, "w") as f:
+            f.write(SRC)
+        csrc = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "inquant-open-source_amd", "csrc")
+        try:
+            subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-fPIC", "-shared", "-I", csrc, "-o", out, src],
+                           check=True, capture_output=True, text=True)
+        except FileNotFoundError as e:
+            pytest.skip(f"g++ unavailable: {e}")
+        return ctypes.CDLL(out).ranges
+
+
+def _host_ranges(x, smean, parts, few):
+    n, c = x.shape
+    x, smean = np.ascontiguousarray(x, F), np.ascontiguousarray(smean, F)
+    out = [np.empty(c, t) for t in (F, F, np.uint64, np.uint64, np.uint8)]
+    _host()(*(ctypes.c_void_p(a.ctypes.data) for a in (x, smean)), ctypes.c_int64(n), ctypes.c_int64(c), parts, int(few),
+            *(ctypes.c_void_p(a.ctypes.data) for a in out))
+    return out
 
 
 @pytest.mark.parametrize("n", [1, 2, 3, 17, 256, 4096, 32768])
@@ -33,17 +78,72 @@ def test_error_range_encloses_the_sequential_pass(n):
     rng = np.random.default_rng(n)
     c = 48
     base = rng.standard_normal((n, c))
+    steps = rng.uniform(1, 2, c).astype(F)
     rows = [base, base * 1e-3 + 5.0, base * 2.0 ** rng.integers(-60, 60, c), np.exp(6 * base), base * 1e-30,
             np.full((n, c), 1.0 / 3.0) + 1e-6 * (np.arange(n) % 2)[:, None], np.zeros((n, c)),
-            np.where(np.arange(n)[:, None] == n - 1, 1e4, base), np.sort(base, 0), 1e18 * base, 3e38 * np.tanh(base)]
+            np.where(np.arange(n)[:, None] == n - 1, 1e4, base), np.sort(base, 0), 1e18 * base, 3e38 * np.tanh(base),
+            # means halfway between two floats, where the sums and the chain may round apart
+            np.where(rng.permuted(np.repeat(np.arange(n)[:, None] % 2, c, 1), axis=0), steps, np.nextafter(steps, F(8)))]
     for x in rows:
         for y in (x.astype(F), synth.bf16_round(x.astype(F))):
             with np.errstate(over="ignore", invalid="ignore"):
                 sal, smean, err, amax = oracle.k4_stats(y, 8, True)
-                lo, hi = _err_range(y, smean)
                 ok = np.isfinite(smean)
-                assert (lo <= hi)[ok].all()
-                assert ((lo <= err) & (err <= hi))[ok].all()
+                for parts in (1, 2, 7, 64):
+                    lo, hi, _, _, _ = _host_ranges(y, smean, parts, False)
+                    assert (lo <= hi)[ok].all()
+                    assert ((lo <= err) & (err <= hi))[ok].all()
+
+
+@pytest.mark.parametrize("n", [2, 5, 100, 256])
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+def test_constant_channels_of_16_bit_values_are_exact(n, kind):
+    # values of every exponent, subnormal ones too; one token of every second channel is the next value of the type
+    rng = np.random.default_rng(n)
+    c = 400
+    if kind == "f16":
+        v = rng.integers(0, 0x7bff, c).astype(np.uint16)
+        to = lambda u: u.view(np.float16).astype(F)
+    else:
+        v = rng.integers(0, 0x7f7f, c).astype(np.uint16)
+        to = lambda u: (u.astype(np.uint32) << 16).view(F)
+    v[:6] = (0, 1, 2, 0x0400, 0x7bfe if kind == "f16" else 0x7f7e, 0x3c00)
+    x = np.repeat(v[None], n, 0)
+    x[rng.integers(0, n, c // 2), np.arange(1, c, 2)] += 1
+    x = to(x) * np.where(np.arange(c) % 3 == 0, F(-1), F(1))
+    constant = (x == x[0]).all(0)
+    assert constant[::2].all() and not constant[1::2].any()
+    sal, smean, err, amax = oracle.k4_stats(x, 8, True)
+    for parts in (1, 2):
+        lo, hi, _, _, same = _host_ranges(x, smean, parts, True)
+        np.testing.assert_array_equal(same.astype(bool), constant)
+        with np.errstate(over="ignore", invalid="ignore"):
+            ok = np.isfinite(smean)
+            assert (lo == err)[constant & ok].all() and (hi == err)[constant & ok].all()
+            assert ((lo <= err) & (err <= hi))[ok].all()
+
+
+@pytest.mark.parametrize("n", [40, 256, 3000])
+def test_certain_pools_are_the_sequential_passes(n):
+    # whenever the enclosures settle a pool, it is the one of the sequential errors; ordinary rows settle, near ties do not
+    rng = np.random.default_rng(n)
+    c = 64
+    settled = {True: 0, False: 0}
+    for i in range(60):
+        near = i % 2 == 1
+        x = np.ones((n, c)) if near else rng.standard_normal((n, c))
+        if near:
+            x[1 + 8 * rng.integers(0, (n - 1) // 8, c), np.arange(c)] += 2.0 ** -7
+        x = x.astype(F)
+        sal, smean, err, amax = oracle.k4_stats(x, 8, True)
+        lo, hi, lo_key, hi_key, _ = _host_ranges(x, smean, 2, False)
+        for count in (1, 8, 31):
+            pool = np.argsort(lo_key)[:count]
+            rest = np.setdiff1d(np.arange(c), pool)
+            if hi_key[pool].max() < lo_key[rest].min():
+                settled[near] += 1
+                assert set(pool) == set(np.argsort(err, kind="stable")[:count])
+    assert settled[False] == 90 and settled[True] < 45
 
 
 def _check(x, stride, frac, policy):
@@ -150,7 +250,6 @@ def test_blocks_with_tied_errors(T, dtype):
 
 def _uncertain(encode):
     """Rows of encode() that took the sequential pass."""
-    import ctypes
     from inquant import _native
 
     def count():
