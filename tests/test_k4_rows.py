@@ -311,3 +311,15 @@ def test_pages_of_repeated_tokens_need_no_sequential_pass(block):
     got = []
     assert _uncertain(lambda: got.append(pack_pages(xt, xt, PageLayout(block, 2)))) == 0
     np.testing.assert_array_equal(got[0].cpu().numpy(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 2, 31, 33, 255, 256])
+@pytest.mark.parametrize("policy", ["neighbors", "min_error"])
+def test_tile_statistics_of_either_policy(T, policy):
+    # every channel's largest magnitude in another token: both halves of the tokens, sampled or not, the last one too
+    x = synth.normal(T, (1, 2, T, 128))
+    x[0, :, (np.arange(128) * 37 + T - 1) % T, np.arange(128)] = (50 + np.arange(128) % 7)[:, None] * np.array([1, -1])
+    xt = torch.from_numpy(x).cuda()
+    assert _uncertain(lambda: _check(xt.bfloat16(), 8, 0.125, policy)) == 0
+    assert _uncertain(lambda: _check(xt.half(), 3, 0.5, policy)) == 0
