@@ -261,6 +261,10 @@ __device__ __forceinline__ int load_desc(const void *p, int64_t i, int bytes)
 }
 
 // One workgroup per (row, token); roles are rebuilt per workgroup in LDS.
+// PLACED: the rows go to their places of a dense history; a tensor of its own
+// needs no division for that (rows of 2000 x 4 x 16 tokens of 66 channels: 116
+// us with it in every workgroup, 102 without).
+template <bool PLACED>
 __global__ __launch_bounds__(V_THREADS) void k4_decode_kernel(KDecArgs a)
 {
     __shared__ int16_t s_role[1024];
@@ -288,7 +292,7 @@ __global__ __launch_bounds__(V_THREADS) void k4_decode_kernel(KDecArgs a)
         } else {
             v = __fmul_rn((float)(slot - 8), a.scales[row * a.D + c]);
         }
-        iq_store_as(a.out, out_row(a, row) + (rt - row * a.T) * a.D + c, v, a.out_dt);
+        iq_store_as(a.out, (PLACED ? out_row(a, row) + (rt - row * a.T) * a.D : rt * a.D) + c, v, a.out_dt);
     }
 }
 
@@ -678,7 +682,8 @@ extern "C" int iq_k4_dequantize_into(const uint8_t *payload, const float *scales
         IQ_CHECK_LAUNCH("k4_decode_words");
         return IQ_OK;
     }
-    hipLaunchKernelGGL(k4_decode_kernel, dim3((unsigned)(rows * T)), block, 0, st, a);
+    if (H == 1 && out_sb == T * D) hipLaunchKernelGGL(k4_decode_kernel<false>, dim3((unsigned)(rows * T)), block, 0, st, a);
+    else hipLaunchKernelGGL(k4_decode_kernel<true>, dim3((unsigned)(rows * T)), block, 0, st, a);
     IQ_CHECK_LAUNCH("k4_decode_kernel");
     return IQ_OK;
 }
