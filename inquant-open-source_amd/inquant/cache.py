@@ -531,9 +531,11 @@ class InQuantCache(_HFCache):
 
     def _position_check(self, position: torch.Tensor, start: int) -> None:
         """Synchronous comparison with start, start + 1, ... (raises before any
-        change), a mismatch still pending from an earlier step included."""
+        change), a mismatch still pending from an earlier step included.  A new
+        cache's first positions are copied to the host: making its flag words
+        takes longer (a first update of 200 tokens: 85 us, 92 with them)."""
         flags = self._flags
-        if _launches(position) and (flags is None or flags.device == position.device):
+        if _launches(position) and (start if flags is None else flags.device == position.device):
             self._position_mismatch(position, start)
             bad = bool(self._flags.tolist()[_POSITION_BAD])
         else:
@@ -551,12 +553,10 @@ class InQuantCache(_HFCache):
     def update(self, key_states, value_states, layer_idx, cache_kwargs=None, *args, **kwargs):
         """Store new tokens; return the layer's full K/V (the inputs themselves
         on the first call, else dequantized history ++ the new tokens)."""
-        if not key_states.is_cuda or _launches(key_states):
-            return self._update(key_states, value_states, layer_idx, cache_kwargs)
-        with torch.cuda.device(key_states.device):
-            return self._update(key_states, value_states, layer_idx, cache_kwargs)
-
-    def _update(self, key_states, value_states, layer_idx, cache_kwargs):
+        device = key_states.get_device()        # -1 on the CPU
+        if device >= 0 and device != torch._C._cuda_getDevice():
+            with torch.cuda.device(device):
+                return InQuantCache.update(self, key_states, value_states, layer_idx, cache_kwargs)
         layer, position = self._check(key_states, value_states, layer_idx, cache_kwargs)
         start = 0 if layer is None else layer.seq_length
         deferred = (position is not None and position.device == key_states.device and _launches(position)
@@ -589,12 +589,10 @@ class InQuantCache(_HFCache):
 
         Blocks sealed by this append are attended from the next step on
         (cache.py:242-269)."""
-        if not key_states.is_cuda or _launches(key_states):
-            return self._append(key_states, value_states, layer_idx, cache_kwargs)
-        with torch.cuda.device(key_states.device):
-            return self._append(key_states, value_states, layer_idx, cache_kwargs)
-
-    def _append(self, key_states, value_states, layer_idx, cache_kwargs) -> PackedAttentionView:
+        device = key_states.get_device()        # -1 on the CPU
+        if device >= 0 and device != torch._C._cuda_getDevice():
+            with torch.cuda.device(device):
+                return InQuantCache.append_for_attention(self, key_states, value_states, layer_idx, cache_kwargs)
         layer, position = self._check(key_states, value_states, layer_idx, cache_kwargs)
         if layer is None or key_states.shape[2] != 1:
             raise ValueError("append_for_attention requires one new token after an existing prefill")
@@ -827,7 +825,7 @@ class InQuantCache(_HFCache):
         layer = self._layers.get(layer_idx)
         if layer is None:
             raise KeyError(f"No cached layer {layer_idx}")
-        if layer.device.type != "cuda" or layer.device.index == torch.cuda.current_device():
+        if layer.device.type != "cuda" or layer.device.index == torch._C._cuda_getDevice():
             return self._dense(layer)
         with torch.cuda.device(layer.device):
             return self._dense(layer)

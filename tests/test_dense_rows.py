@@ -99,7 +99,7 @@ def test_every_launch_of_the_cache_runs_on_the_gpu_of_its_tensors(monkeypatch, v
             return getattr(lib, name)
 
     row = _native.tail_append_row
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: current[0])        # torch.cuda.current_device() too
     monkeypatch.setattr(torch.cuda, "device", Switch)
     monkeypatch.setattr(_native, "lib", Spy)
     monkeypatch.setattr(_native, "tail_append_row", lambda *args: (launches.append(("append", current[0])), row(*args))[1])
@@ -129,6 +129,22 @@ def test_positions_are_checked_before_a_sealing_update_changes_the_layer(dtype):
     assert cache.get_seq_length() == 60 and cache._layers[0].key_blocks[0] is blocks[0]
     with pytest.raises(ValueError, match="contiguous append"):
         InQuantCache(cache.config).update(k, k, 0, {"cache_position": wrong})
+
+
+def test_first_positions_of_a_new_cache_make_no_flag_words():
+    from inquant.cache import CacheConfig, InQuantCache
+    k = torch.randn(1, 2, 9, 64, device="cuda").bfloat16()
+    pos = torch.arange(9, device="cuda")
+    cache = InQuantCache(CacheConfig(block_size=8, residual_length=4, sink_tokens=2))
+    for wrong in (pos[1:6], pos[:5].flip(0), pos[:5] + 2 ** 40):
+        with pytest.raises(ValueError, match="contiguous append"):
+            cache.update(k[:, :, :5], k[:, :, :5], 0, {"cache_position": wrong})
+    cache.update(k[:, :, :5], k[:, :, :5], 0, {"cache_position": pos[:5]})
+    assert cache._flags is None
+    with pytest.raises(ValueError, match="contiguous append"):
+        cache.update(k[:, :, 5:7], k[:, :, 5:7], 0, {"cache_position": pos[6:8]})
+    cache.update(k[:, :, 5:7], k[:, :, 5:7], 0, {"cache_position": pos[5:7]})
+    assert cache.get_seq_length() == 7 and not any(cache._flags.tolist())
 
 
 def test_positions_come_before_the_errors_of_a_sealing_update():
