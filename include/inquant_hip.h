@@ -393,6 +393,17 @@ int iq_prefill_attention(const void *q, const void *k, const void *v, int dtype,
                          void *out, int64_t o_st, int64_t o_sh, int out_dtype, void *stream);
 
 /*
+ * The same with the tokens of all sequences together (or a bound on them; 0:
+ * unknown), by which the order of the work is chosen; the results do not
+ * depend on it.
+ */
+int iq_prefill_attention_tokens(const void *q, const void *k, const void *v, int dtype, int64_t q_st, int64_t q_sh,
+                                int64_t k_st, int64_t k_sh, int64_t v_st, int64_t v_sh, const int32_t *cu_seqlens,
+                                int64_t n_seq, int64_t max_seqlen, int64_t tokens, int64_t Hq, int64_t H,
+                                int64_t head_dim, float scale, void *out, int64_t o_st, int64_t o_sh, int out_dtype,
+                                void *stream);
+
+/*
  * Dense tail append of a cache layer.  buf holds [2 (keys, values), H,
  * capacity, D] elements of elem_bytes (element strides buf_kv, buf_h,
  * buf_t); k / v hold n_new (<= 64) rows per head (element strides: head,

@@ -1053,8 +1053,8 @@ __global__ __launch_bounds__(K4_THREADS) void k4_quantize_rows(K4Args a, int64_t
 // ---------------------------------------------------------------------------
 // Tile encoder for the cache shapes: D = 128, 16-bit input, T <= 256 tokens,
 // channel-contiguous rows.  The block streams through LDS in 32-token chunks
-// (double-buffered, 16-byte loads, three chunks in flight while the current
-// one is consumed), twice:
+// (16-byte loads; sealed blocks by direct loads with three chunks in flight
+// while one is consumed, others double-buffered through registers), twice:
 //   pass 1  thread (half, channel) sums x and x^2 of every other token in
 //           fp64 (min_error only) and takes amax and finiteness as an integer
 //           max of the 16-bit magnitudes; one half also adds the sampled
@@ -1168,8 +1168,7 @@ __device__ __forceinline__ void k4_tile_body(const K4Args &a, int64_t b, int64_t
 
     // chunk staging: thread tid moves segments tid and tid + 256 (row i / 16,
     // 8 channels at 8 (i % 16)); rows past T are clamped copies, never read.
-    // Three chunks stay in flight in registers (about 24 KiB per block), which
-    // is what covers the load latency while every block streams at once.
+    // The next chunk is in flight in registers while one is processed.
     u32x4_t seg[KPF][2];
     auto load_chunk = [&](int ch, u32x4_t (&sg)[2]) {
 #pragma unroll

@@ -26,8 +26,8 @@
 // stages of row-major K and V with XOR-swizzled 16-byte chunks; the V
 // operand of O^T = V^T P^T comes out of LDS already transposed
 // (ds_read_b64_tr_b16); one barrier per tile.  Masks only on the diagonal
-// and last tiles; query tiles longest-first, each XCD on a contiguous range
-// of (query head, tile) items.  184 VGPRs: two wavefronts per SIMD.
+// and last tiles; query tiles longest-first, spread evenly over the XCDs.
+// 184 VGPRs: two wavefronts per SIMD.
 #include "decode_common.h"
 
 namespace {
@@ -46,7 +46,7 @@ struct PrefillArgs {
     void *out;
     int64_t q_st, q_sh, k_st, k_sh, v_st, v_sh, o_st, o_sh;   // element strides (token, head)
     const int32_t *cu;                                        // [n_seq + 1] token offsets
-    int tiles, span, n_seq, Hq;                               // query tiles per sequence, places per group, sequences, query heads
+    int tiles, span, share, n_seq, Hq;                        // query tiles per sequence, places per group, an XCD's items of one, sequences, query heads
     int G;
     float c_log2;                                             // softmax scale * log2(e)
     int odt;
@@ -115,16 +115,29 @@ __global__ __launch_bounds__(NT, 2) void prefill_attn(PrefillArgs a)
     // of `span` places an XCD takes the same share of neighbouring heads in
     // every sequence (span Hq / 8 items), so the work of the XCDs is even and
     // an XCD's resident workgroups read the K/V of a KV head at about the same
-    // time, out of its own L2.  8K causal, 28 query heads: 516 us (933 TFLOP/s)
-    // with a contiguous range of (head, tile) items per XCD, where four of the
-    // XCDs had 15% more work than the others and ended on long tiles, 468 (1028)
-    // with these; seven prompts of up to 4.1K tokens, 32 heads: 293 and 281.
-    const int share = a.span * a.Hq / 8;
-    const int j = (int)(blockIdx.x >> 3), rest = j % (a.n_seq * share);
-    const int at = (int)(blockIdx.x & 7) * share + rest % share;
-    const int seq = rest / share, hq = at / a.span, h = hq / a.G;
-    const int place = a.tiles - 1 - (j / (a.n_seq * share) * a.span + at % a.span);
-    if (place < 0) return;                       // the last group's padding
+    // time, out of its own L2.  8K causal, 28 query heads, eager: 519 us (927
+    // TFLOP/s) with a contiguous range of (head, tile) items per XCD, where
+    // four of the XCDs had 15% more work than the others and ended on long
+    // tiles, 463 (1039) with these; seven prompts of up to 4.1K tokens, 32
+    // heads: 293 and 281.  span = 0 is that contiguous range, a sequence after
+    // the other (blockIdx.y).
+    const int xcd = (int)(blockIdx.x & 7), j = (int)(blockIdx.x >> 3);
+    int seq, hq, place;
+    if (a.span == 0) {
+        const int item = xcd * a.share + j;
+        if (item >= a.tiles * a.Hq) return;      // the slice's padding
+        seq = blockIdx.y;
+        hq = item / a.tiles;
+        place = a.tiles - 1 - (item - hq * a.tiles);
+    } else {
+        const int per = a.n_seq * a.share, group = j / per, rest = j - group * per;
+        seq = rest / a.share;
+        const int at = xcd * a.share + rest - seq * a.share;
+        hq = at / a.span;
+        place = a.tiles - 1 - (group * a.span + at - hq * a.span);
+        if (place < 0) return;                   // the last group's padding
+    }
+    const int h = hq / a.G;
     const int start = a.cu[seq], len = a.cu[seq + 1] - start;
     const int q0 = place * QT;
     if (q0 >= len) return;                       // uniform: no barrier is skipped by part of the group
@@ -300,9 +313,9 @@ __global__ __launch_bounds__(NT, 2) void prefill_attn(PrefillArgs a)
 
 }  // namespace
 
-extern "C" int iq_prefill_attention(const void *q, const void *k, const void *v, int dtype, int64_t q_st,
+extern "C" int iq_prefill_attention_tokens(const void *q, const void *k, const void *v, int dtype, int64_t q_st,
                                     int64_t q_sh, int64_t k_st, int64_t k_sh, int64_t v_st, int64_t v_sh,
-                                    const int32_t *cu_seqlens, int64_t n_seq, int64_t max_seqlen, int64_t Hq,
+                                    const int32_t *cu_seqlens, int64_t n_seq, int64_t max_seqlen, int64_t tokens, int64_t Hq,
                                     int64_t H, int64_t head_dim, float scale, void *out, int64_t o_st,
                                     int64_t o_sh, int out_dtype, void *stream)
 {
@@ -314,6 +327,7 @@ extern "C" int iq_prefill_attention(const void *q, const void *k, const void *v,
                  (long long)Hq, (long long)H);
     IQ_CHECK_ARG(n_seq >= 1 && n_seq <= 65535 && max_seqlen >= 1 && max_seqlen <= 0x7fffffffLL - QT,
                  "iq_prefill_attention: bad sequence count or length");
+    IQ_CHECK_ARG(tokens >= 0 && tokens <= (int64_t(1) << 60), "iq_prefill_attention: bad token count");
     // a key tile's rows are addressed by 32-bit byte offsets from its first row
     IQ_CHECK_ARG(k_st >= 0 && v_st >= 0 && k_st < (1LL << 25) && v_st < (1LL << 25),
                  "iq_prefill_attention: token stride too large");
@@ -338,21 +352,45 @@ extern "C" int iq_prefill_attention(const void *q, const void *k, const void *v,
     // six of up to 12K: 3.07, 3.16 and 3.00)
     int64_t span = 1;
     while (span * Hq % 8) span *= 2;
+    // Workgroups past their sequence's end leave at once, and as an XCD deals
+    // its workgroups round-robin over its CUs, the others meet on a part of
+    // them where they stand at a fixed stride.  So the groups are for batches
+    // whose tokens are at least two fifths of what the bound allows (under
+    // that: 8 heads over 8, 200 prompts of 129 tokens bound by 516, 66 us in
+    // contiguous ranges and 209 in groups; eight prompts, one of 4096 tokens,
+    // 81 and 105; above: 28 heads over 4, prompts of 300 to 4000 tokens, 203
+    // and 174) and that have more places than a group (64 prompts of 1 token,
+    // 14 heads: 12.4 us, and 15.8 padded to groups of 4).
     const int64_t least = n_seq == 1 ? 1 : max_seqlen <= 8192 ? 4 : 224;
     if (least == 224 && Hq % 8 == 0) span = tiles;
     while (span * Hq / 8 < least && span < tiles) span *= 2;
-    const int64_t per_seq = (tiles + span - 1) / span * span * Hq;
+    const bool groups = span < tiles && 5 * tokens >= 2 * n_seq * max_seqlen;
+    if (!groups) span = 0;
+    const int64_t share = groups ? span * Hq / 8 : (tiles * Hq + 7) / 8;
+    const int64_t per_seq = groups ? (tiles + span - 1) / span * share * 8 : share * 8;
     constexpr int64_t MOST = 0xffffffffLL / NT;          // workgroups of a launch (2^32 threads)
     IQ_CHECK_ARG(per_seq <= MOST, "iq_prefill_attention: too many query tiles");
-    for (int64_t s0 = 0; s0 < n_seq; s0 += MOST / per_seq) {
-        const int64_t n = n_seq - s0 < MOST / per_seq ? n_seq - s0 : MOST / per_seq;
+    const int64_t most = groups ? MOST / per_seq : n_seq;
+    for (int64_t s0 = 0; s0 < n_seq; s0 += most) {
+        const int64_t n = n_seq - s0 < most ? n_seq - s0 : most;
         PrefillArgs a{(const uint16_t *)q, (const uint16_t *)k, (const uint16_t *)v, out, q_st, q_sh, k_st, k_sh,
-                      v_st, v_sh, o_st, o_sh, cu_seqlens + s0, (int)tiles, (int)span, (int)n, (int)Hq, (int)(Hq / H),
+                      v_st, v_sh, o_st, o_sh, cu_seqlens + s0, (int)tiles, (int)span, (int)share, (int)n, (int)Hq, (int)(Hq / H),
                       scale * 1.44269504088896341f, out_dtype, vec_out};
-        const dim3 grid((unsigned)(per_seq * n)), block(NT);
+        const dim3 grid((unsigned)(groups ? per_seq * n : per_seq), groups ? 1u : (unsigned)n), block(NT);
         if (dtype == IQ_F16) hipLaunchKernelGGL(prefill_attn<true>, grid, block, 0, (hipStream_t)stream, a);
         else hipLaunchKernelGGL(prefill_attn<false>, grid, block, 0, (hipStream_t)stream, a);
     }
     IQ_CHECK_LAUNCH("prefill_attn");
     return IQ_OK;
+}
+
+extern "C" int iq_prefill_attention(const void *q, const void *k, const void *v, int dtype, int64_t q_st, int64_t q_sh,
+                                    int64_t k_st, int64_t k_sh, int64_t v_st, int64_t v_sh, const int32_t *cu_seqlens,
+                                    int64_t n_seq, int64_t max_seqlen, int64_t Hq, int64_t H, int64_t head_dim,
+                                    float scale, void *out, int64_t o_st, int64_t o_sh, int out_dtype, void *stream)
+{
+    // one sequence is as long as its bound; of several nothing is known
+    return iq_prefill_attention_tokens(q, k, v, dtype, q_st, q_sh, k_st, k_sh, v_st, v_sh, cu_seqlens, n_seq, max_seqlen,
+                                       n_seq == 1 && max_seqlen > 0 ? max_seqlen : 0, Hq, H, head_dim, scale, out, o_st,
+                                       o_sh, out_dtype, stream);
 }

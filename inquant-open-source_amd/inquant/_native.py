@@ -87,6 +87,8 @@ _SIGNATURES = {
                                            _f32, _p, _int, _p]),
     "iq_prefill_attention": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64,
                                     _i64, _i64, _f32, _p, _i64, _i64, _int, _p]),
+    "iq_prefill_attention_tokens": (_int, [_p, _p, _p, _int, _i64, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i64, _i64,
+                                           _i64, _i64, _i64, _f32, _p, _i64, _i64, _int, _p]),
     "iq_page_bytes": (_i64, [_i64, _i64]),
     "iq_encode_pages": (_int, [_p, _p, _int, ctypes.POINTER(_i64), ctypes.POINTER(_i64), _i64, _i64, _i64, _p, _i64,
                                _p, _int, _p, _p, _p]),

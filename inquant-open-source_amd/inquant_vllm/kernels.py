@@ -146,9 +146,9 @@ def prefill_attention(query, key, value, cu_seqlens, max_seqlen, scale, output=N
             or output.dtype not in (query.dtype, torch.float32):
         raise ValueError("output must be [tokens, Hq, 128] of the query dtype or float32")
     cu = cu_seqlens.contiguous()
-    nat.check(nat.lib().iq_prefill_attention(
+    nat.check(nat.lib().iq_prefill_attention_tokens(
         query.data_ptr(), key.data_ptr(), value.data_ptr(), nat.dtype_code(query.dtype),
         query.stride(0), query.stride(1), key.stride(0), key.stride(1), value.stride(0), value.stride(1),
-        cu.data_ptr(), cu.numel() - 1, int(max_seqlen), hq, h, 128, float(scale), output.data_ptr(),
+        cu.data_ptr(), cu.numel() - 1, int(max_seqlen), query.shape[0], hq, h, 128, float(scale), output.data_ptr(),
         output.stride(0), output.stride(1), nat.dtype_code(output.dtype), nat.stream_handle(query.device)))
     return output

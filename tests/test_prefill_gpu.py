@@ -156,6 +156,29 @@ def test_prefill_items_of_a_batch_cover_every_sequence(hq, h, lens):
         assert torch.equal(got[a:b], alone)
 
 
+@pytest.mark.parametrize("hq,h", [(1, 1), (8, 8), (12, 4), (14, 2), (28, 4)])
+@pytest.mark.parametrize("lens", [(0, 300, 0, 5, 1100), (129,) * 70, (700, 0) * 33 + (1,), (1, 140, 260) * 85, (130, 2) * 129,
+                                  (0, 0), (513,)])
+@pytest.mark.parametrize("loose", [1, 4])
+def test_prefill_items_under_a_loose_bound(hq, h, lens, loose):
+    # sequences without tokens, more of them than a wavefront's lanes (and than a launch orders by groups), bounds above
+    # the longest: every row is that of the sequence alone, and no other is written
+    from inquant_vllm.kernels import prefill_attention
+    q, k, v = _qkv(hq + len(lens), sum(lens) + 1, hq, h, torch.bfloat16)
+    offsets = [0, *np.cumsum(lens).tolist()]
+    cu = torch.tensor(offsets, dtype=torch.int32, device="cuda")
+    got = prefill_attention(q, k, v, cu, loose * max(1, *lens), 128 ** -0.5, torch.full_like(q, float("nan")))
+    assert got[sum(lens):].isnan().all()
+    for length in sorted(set(lens) - {0}):
+        i = [n for n, x in enumerate(lens) if x == length]
+        for n in {i[0], i[len(i) // 2], i[-1]}:
+            a, b = offsets[n:n + 2]
+            one = torch.tensor([0, b - a], dtype=torch.int32, device="cuda")
+            alone = prefill_attention(q[a:b], k[a:b], v[a:b], one, b - a, 128 ** -0.5, torch.full_like(q[a:b], float("nan")))
+            assert torch.equal(got[a:b], alone)
+    assert not got[:sum(lens)].isnan().any()
+
+
 def test_prefill_rejects_bad_arguments():
     from inquant_vllm import prefill_attention
     q, k, v = _qkv(1, 8, 4, 2, torch.bfloat16)
