@@ -125,8 +125,8 @@ class _BlockFormat:
             elif not isinstance(v, PackedTensor) or v.salient_channels.shape[-1] != self.salient:
                 raise ValueError("All InQuant V blocks must share the salient-channel count")
         index = self.device.index
-        for _, packed, _, _ in (*keys, *values):
-            for t in packed.tensors.values():
+        for run in (*keys, *values):
+            for t in run[1].tensors.values():
                 if t.get_device() != index:
                     raise ValueError("All packed tensors must share the same CUDA device")
         if self.salient > 64:
@@ -147,6 +147,12 @@ def _column(runs, name: str) -> list:
         else:
             out.extend(range(base + first * step, base + (first + count) * step, step))
     return out
+
+
+def _block_addresses(k, v) -> tuple:
+    """The addresses of a block with 2/4-bit values, in pointer-table column order."""
+    return (k.payload.data_ptr(), k.scales.data_ptr(), k.padding.data_ptr(), v.payload.data_ptr(),
+            v.scales.data_ptr(), v.offsets.data_ptr(), k.salient_channels.data_ptr(), k.donor_channels.data_ptr())
 
 
 def _block_columns(keys, values, k4_values: bool) -> list:
@@ -197,11 +203,21 @@ class _Descriptors:
         if self.k4_values:
             self.value_map = regrow(self.value_map, (grown, *self.value_map.shape[1:]))
 
-    def grow_run(self, first: int, columns, fmt: _BlockFormat) -> None:
-        """Extend the fixed-stride run over the new blocks while they continue it."""
-        if not self.run_open or fmt.value_bits == 0:
-            self.run_open = False
-            return
+    def grow_run(self, first: int, rows, fmt: _BlockFormat) -> None:
+        """Extend the fixed-stride run over new blocks, an iterable of their
+        addresses, while they continue it."""
+        run, steps = self.run, _field_bytes(fmt)
+        for i, addr in enumerate(rows):
+            if run.blocks == 0 and first + i == 0:
+                run.base[:] = addr
+            elif run.blocks != first + i or any(a != base + run.blocks * step
+                                                for a, base, step in zip(addr, run.base, steps)):
+                self.run_open = False
+                return
+            run.blocks += 1
+
+    def grow_run_columns(self, first: int, columns, fmt: _BlockFormat) -> None:
+        """The same for the addresses by field."""
         run, count = self.run, len(columns[0])
         if run.blocks == 0 and first == 0:
             run.base[:] = [c[0] for c in columns[:_COLUMNS]]
@@ -214,14 +230,34 @@ class _Descriptors:
         run.blocks += more
         self.run_open = more == count
 
-    def write(self, first: int, keys, values, fmt: _BlockFormat, stream: int) -> None:
-        columns = _block_columns(keys, values, self.k4_values)
-        self.grow_run(first, columns, fmt)
-        count = len(columns[0])
+    def write(self, first: int, keys, values, plain: bool, fmt: _BlockFormat, stream: int) -> None:
+        """The rows of new blocks, runs of them (_batch_runs).  ``plain``: all
+        are blocks of their own (a seal's), whose addresses are read one by one:
+        one of them extends a state in 11 us, 25 by way of the columns; 127 of a
+        batch in 116 by the columns, 545 one by one."""
+        self.run_open = self.run_open and fmt.value_bits != 0
+        count = len(keys) if plain else sum(run[3] for run in keys)
         rows = (nat.BlockPtrs * count)()
-        words = memoryview(rows).cast("B").cast("Q")
-        for f, column in enumerate(columns):
-            words[f::len(columns)] = array("Q", column)
+        if plain:
+            keys, values = [run[0] for run in keys], [run[0] for run in values]
+            if self.run_open:
+                self.grow_run(first, map(_block_addresses, keys, values), fmt)
+            for row, k, v in zip(rows, keys, values):
+                row.k_payload, row.k_scales, row.k_padding = k.payload.data_ptr(), k.scales.data_ptr(), k.padding.data_ptr()
+                row.k_src, row.k_don = k.salient_channels.data_ptr(), k.donor_channels.data_ptr()
+                row.v_payload, row.v_scales = v.payload.data_ptr(), v.scales.data_ptr()
+                if self.k4_values:
+                    row.v_offsets = v.padding.data_ptr()
+                    row.v_src, row.v_don = v.salient_channels.data_ptr(), v.donor_channels.data_ptr()
+                else:
+                    row.v_offsets = v.offsets.data_ptr()
+        else:
+            columns = _block_columns(keys, values, self.k4_values)
+            if self.run_open:
+                self.grow_run_columns(first, columns, fmt)
+            words = memoryview(rows).cast("B").cast("Q")
+            for f, column in enumerate(columns):
+                words[f::len(columns)] = array("Q", column)
         nat.check(nat.lib().iq_decode_append(
             self.tables.data_ptr(), self.key_map.data_ptr(),
             self.value_map.data_ptr() if self.k4_values else None, first, count, rows, fmt.heads,
@@ -316,13 +352,15 @@ class PackedDecodeState:
                 raise ValueError("All packed K/V blocks must share shape and salient-channel count")
         stream = self._pin.check(fmt.device)
         new_keys, new_values = tuple(key_blocks[have:]), tuple(value_blocks[have:])
-        key_runs, value_runs = list(_batch_runs(new_keys)), list(_batch_runs(new_values))
+        plain = all([getattr(b, "_batch", None) is None for b in new_keys + new_values])
+        key_runs, value_runs = ([(b, b, 0, 1) for b in new] if plain else list(_batch_runs(new))
+                                for new in (new_keys, new_values))
         fmt.admit(key_runs, value_runs)
         if not have:      # also after dense-only steps, whose tables are of no format
             self._desc = _Descriptors(fmt.device, fmt.heads, fmt.value_bits == 0)
         self._format = fmt
         self._desc.reserve(have, len(key_blocks))
-        self._desc.write(have, key_runs, value_runs, fmt, stream)
+        self._desc.write(have, key_runs, value_runs, plain, fmt, stream)
         # only the new blocks are added (the held prefix is identical): no
         # pass over the whole history beyond the identity check
         self._keys.extend(new_keys)

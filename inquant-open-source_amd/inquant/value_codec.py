@@ -12,9 +12,10 @@ from dataclasses import dataclass
 import torch
 
 from . import _native as nat
-from .codec import _BlockFields, _per_block, _view_nbytes
+from .codec import _BlockFields, _fields_on_demand, _per_block, _view_nbytes
 
 
+@_fields_on_demand
 @dataclass(frozen=True)
 class PackedValues(_BlockFields):
     payload: torch.Tensor
