@@ -40,7 +40,8 @@
  *   iq_unpack_pages     extensions/vllm/src/inquant_vllm/layout.py:84-100 unpack_pages_reference
  *   iq_paged_decode     extensions/vllm/src/inquant_vllm/kernels.py:66-88 paged_decode
  *   iq_prefill_attention extensions/vllm/src/inquant_vllm/backend.py:139-144
- *                       (flash_attn_varlen_func, causal prefill on exact K/V)
+ *                       (flash_attn_varlen_func, causal prefill on exact K/V);
+ *                       iq_prefill_attention_tokens, the same with the token count
  *   iq_tail_append      src/inquant/cache.py:256-259,283-286 (the dense tail
  *                       concatenation of append_for_attention / _append)
  */
