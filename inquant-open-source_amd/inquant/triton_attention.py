@@ -109,14 +109,16 @@ class _BlockFormat:
     def same(self, other: "_BlockFormat") -> bool:
         return all(getattr(self, f) == getattr(other, f) for f in self.__slots__)
 
-    def admit(self, keys, values) -> None:
-        """Raise the reference's errors for blocks (runs of them, _batch_runs)
-        that break the layout."""
-        for block, k, _, _ in keys:
+    def admit(self, keys, values, plain: bool) -> None:
+        """Raise the reference's errors for blocks that break the layout: blocks
+        of their own (``plain``) or runs of blocks (_batch_runs)."""
+        firsts = zip(keys, keys) if plain else [run[:2] for run in keys]
+        for block, k in firsts:
             if (not isinstance(k, PackedTensor) or block.shape != (1, self.heads, self.tokens, 128)
                     or k.salient_channels.shape[-1] != self.salient):
                 raise ValueError("All packed K/V blocks must share shape and salient-channel count")
-        for block, v, _, _ in values:
+        firsts = zip(values, values) if plain else [run[:2] for run in values]
+        for block, v in firsts:
             if block.shape != (1, self.heads, self.tokens, 128):
                 raise ValueError("All packed blocks must share shape")
             if self.value_bits:
@@ -125,8 +127,8 @@ class _BlockFormat:
             elif not isinstance(v, PackedTensor) or v.salient_channels.shape[-1] != self.salient:
                 raise ValueError("All InQuant V blocks must share the salient-channel count")
         index = self.device.index
-        for run in (*keys, *values):
-            for t in run[1].tensors.values():
+        for packed in (*keys, *values) if plain else [run[1] for run in (*keys, *values)]:
+            for t in packed.tensors.values():
                 if t.get_device() != index:
                     raise ValueError("All packed tensors must share the same CUDA device")
         if self.salient > 64:
@@ -231,15 +233,14 @@ class _Descriptors:
         self.run_open = more == count
 
     def write(self, first: int, keys, values, plain: bool, fmt: _BlockFormat, stream: int) -> None:
-        """The rows of new blocks, runs of them (_batch_runs).  ``plain``: all
-        are blocks of their own (a seal's), whose addresses are read one by one:
-        one of them extends a state in 11 us, 25 by way of the columns; 127 of a
-        batch in 116 by the columns, 545 one by one."""
+        """The rows of new blocks: blocks of their own (``plain``, a seal's),
+        whose addresses are read one by one, or runs of blocks (_batch_runs).
+        One of its own extends a state in 11 us, 25 by way of the columns; 127 of
+        a batch in 116 by the columns, 545 one by one."""
         self.run_open = self.run_open and fmt.value_bits != 0
         count = len(keys) if plain else sum(run[3] for run in keys)
         rows = (nat.BlockPtrs * count)()
         if plain:
-            keys, values = [run[0] for run in keys], [run[0] for run in values]
             if self.run_open:
                 self.grow_run(first, map(_block_addresses, keys, values), fmt)
             for row, k, v in zip(rows, keys, values):
@@ -353,14 +354,13 @@ class PackedDecodeState:
         stream = self._pin.check(fmt.device)
         new_keys, new_values = tuple(key_blocks[have:]), tuple(value_blocks[have:])
         plain = all([getattr(b, "_batch", None) is None for b in new_keys + new_values])
-        key_runs, value_runs = ([(b, b, 0, 1) for b in new] if plain else list(_batch_runs(new))
-                                for new in (new_keys, new_values))
-        fmt.admit(key_runs, value_runs)
+        keys, values = (new_keys, new_values) if plain else map(list, map(_batch_runs, (new_keys, new_values)))
+        fmt.admit(keys, values, plain)
         if not have:      # also after dense-only steps, whose tables are of no format
             self._desc = _Descriptors(fmt.device, fmt.heads, fmt.value_bits == 0)
         self._format = fmt
         self._desc.reserve(have, len(key_blocks))
-        self._desc.write(have, key_runs, value_runs, plain, fmt, stream)
+        self._desc.write(have, keys, values, plain, fmt, stream)
         # only the new blocks are added (the held prefix is identical): no
         # pass over the whole history beyond the identity check
         self._keys.extend(new_keys)
